@@ -18,6 +18,7 @@
 
 #include "odis.h"
 #include "odis_kernels.hpp"
+#include "odis_resident.hpp"
 
 namespace odis {
 
@@ -2105,6 +2106,33 @@ uint64_t hilbert3(uint32_t X0, uint32_t X1, uint32_t X2, int bits) {
 
 }  // namespace
 
+// Launches of k_resident: its patches and workspace on the device, and the
+// launches not yet known to have run (the host looks at `status` whenever it
+// waits for the stream anyway).
+struct ResDev {
+  int W = 0;                   // patches per instance (0: not set up)
+  int variant = 0, ipl = 0;    // kernel variant, instances at a time
+  int max_cells = 0, max_face = 0, max_bnd = 0, slots = 0;
+  const int *cptr = nullptr, *fptr = nullptr, *bptr = nullptr, *cell = nullptr, *face = nullptr, *fcell = nullptr;
+  const int *bface = nullptr, *bcell = nullptr, *bhalo = nullptr, *bpeer = nullptr;
+  const unsigned short *cyc = nullptr;
+  uint4v *mail = nullptr;
+  unsigned long long *ctl = nullptr;
+  double *part = nullptr;
+  int chunk = 0;               // steps per launch at most
+  unsigned *status = nullptr;  // pinned host memory
+  unsigned seq = 0, launch = 0;
+  unsigned long long arrived = 0;
+  int off = 0;                 // not usable on this context (or taken back once)
+  std::vector<void *> allocs;
+  struct Pending {
+    unsigned launch;
+    long long n0;
+    int cur;
+  };
+  std::vector<Pending> pending;
+};
+
 // Event pairs (start, end) recorded for the kernels of sampled steps.
 struct ChunkEvents {
   std::vector<int> mom;   // momentum kernel (k_face, or the one-kernel k_step) of each sampled step
@@ -2142,8 +2170,12 @@ struct odis_ctx {
   void *il_buf = nullptr;      // interleaved v[2], eta[2], ring_v, ring_e, ts[2]
   int il_fresh = 0;            // the interleaved copy holds the current state
   int std_fresh = 1;           // the instance-major arrays hold the current state
+  // resident launches (many steps per launch, odis_resident.hpp)
+  int res_opt = 1;             // ODIS_OPT_RESIDENT: 0 off, 1 automatic, > 1 that many patches per instance
+  ResDev res;
   std::string one_kernel_why;
   std::vector<int> gi_host, cyc_host;  // device-order face cells and cell cycles, to rebuild patches
+  std::vector<float> cell_xyz;         // [N][3] unit vectors of the device cells, for the resident patches
   long long step = 0;          // next step index n, shared by all instances
   long long series_lo = 0;     // first step of the series ring written since the last set_state
   // orbit statistics: FP64 state snapshot [B][E + N] per instance at its last
@@ -2463,6 +2495,16 @@ static int build_compact_ops(odis_ctx *ctx, Ops<T> &o, const CompactHost &h) {
   return ODIS_OK;
 }
 
+template <typename T>
+static int res_setup(odis_ctx *ctx);
+static bool res_wanted(const odis_ctx *ctx);
+
+static void res_free(odis_ctx *ctx) {
+  for (void *p : ctx->res.allocs) (void)hipFree(p);
+  if (ctx->res.status) (void)hipHostFree(ctx->res.status);
+  ctx->res = ResDev();
+}
+
 extern "C" int odis_destroy(odis_ctx *ctx) {
   if (!ctx) return ODIS_E_INVALID;
   if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
@@ -2474,6 +2516,7 @@ extern "C" int odis_destroy(odis_ctx *ctx) {
     if (ctx->coef_ev[k]) (void)hipEventDestroy(ctx->coef_ev[k]);
     if (ctx->coef_host[k]) (void)hipHostFree(ctx->coef_host[k]);
   }
+  res_free(ctx);
   for (void *p : ctx->allocs) (void)hipFree(p);
   for (void *p : ctx->rbf_allocs) (void)hipFree(p);
   for (void *p : ctx->ll_allocs) (void)hipFree(p);
@@ -2529,27 +2572,33 @@ static int create_impl(const odis_mesh_desc *m, const odis_params *params, int n
   ctx->params.assign(params, params + n_inst);
   ctx->energy_quad = params[0].friction == ODIS_QUADRATIC;
   ctx->quad_drag = params[0].quad_drag != 0;
-  ctx->init_hist_v.assign(n_inst, std::vector<double>(size_t(3) * E, 0.0));
-  ctx->init_hist_e.assign(n_inst, std::vector<double>(size_t(3) * N, 0.0));
+  ctx->init_hist_v.resize(n_inst);  // empty: zeros
+  ctx->init_hist_e.resize(n_inst);
   ctx->cell_lat.assign(m->cell_lat, m->cell_lat + N);
   ctx->cell_lon.assign(m->cell_lon, m->cell_lon + N);
 
   // -- locality renumbering: cells along a 3-D Hilbert curve, faces by the
   //    device ranks of their two cells
   std::vector<std::pair<uint64_t, int>> ck(N);
+  std::vector<float> xyz(size_t(3) * N);
   for (int i = 0; i < N; i++) {
     const double la = m->cell_lat[i], lo = m->cell_lon[i];
     const double x = std::cos(la) * std::cos(lo), y = std::cos(la) * std::sin(lo), z = std::sin(la);
     const double s = double((1u << 20) - 1);
     auto q = [&](double v) { return uint32_t(std::lround((v + 1.0) * 0.5 * s)); };
     ck[i] = {hilbert3(q(x), q(y), q(z), 20), i};
+    xyz[size_t(3) * i] = float(x);
+    xyz[size_t(3) * i + 1] = float(y);
+    xyz[size_t(3) * i + 2] = float(z);
   }
   std::stable_sort(ck.begin(), ck.end());
   ctx->cell_perm.resize(N);
   ctx->cell_inv.resize(N);
+  ctx->cell_xyz.resize(size_t(3) * N);
   for (int r = 0; r < N; r++) {
     ctx->cell_inv[r] = ck[r].second;
     ctx->cell_perm[ck[r].second] = r;
+    for (int d = 0; d < 3; d++) ctx->cell_xyz[size_t(3) * r + d] = xyz[size_t(3) * ck[r].second + d];
   }
   std::vector<std::pair<std::pair<int, int>, int>> fk(E);
   for (int e = 0; e < E; e++) {
@@ -2726,6 +2775,7 @@ static int create_impl(const odis_mesh_desc *m, const odis_params *params, int n
     if (he == hipSuccess) he = hipDeviceSynchronize();
     if (he != hipSuccess) rc = fail(ctx, ODIS_E_HIP, hipGetErrorString(he));
   }
+  if (!rc && res_wanted(ctx)) rc = precision == ODIS_FP64 ? res_setup<double>(ctx) : res_setup<float>(ctx);
   *building = nullptr;
   if (rc) {
     const std::string msg = ctx->err;
@@ -2760,6 +2810,7 @@ extern "C" const char *odis_last_error(const odis_ctx *ctx) {
 // 36-65); after step m >= 1 it holds (f_m, f_m, f_{m-1}), except after an
 // Euler step 0 (f_0, ds1 as set, f_0).  set/get translate between the two.
 
+static int res_settle(odis_ctx *ctx);  // resident launches known to have run (or their steps run again)
 static int il_out_any(odis_ctx *ctx);  // the instance-major arrays up to date (batches held interleaved)
 
 template <typename T>
@@ -2846,13 +2897,13 @@ static int get_state_t(odis_ctx *ctx, Ops<T> &o, int b, double *v, double *dv, d
     for (int r = 0; r < M; r++) {
       const int i = inv[r];
       if (k == 0) {  // no step since set_state: the history as set
-        for (int q = 0; q < 3; q++) ds[3 * i + q] = keep[3 * i + q];
+        for (int q = 0; q < 3; q++) ds[3 * i + q] = keep.empty() ? 0.0 : keep[3 * i + q];
         continue;
       }
       const double last = double(all[size_t((k - 1) % 3) * M + r]);
       ds[3 * i + 0] = last;
       if (k == 1 && !load) {
-        ds[3 * i + 1] = keep[3 * i + 1];
+        ds[3 * i + 1] = keep.empty() ? 0.0 : keep[3 * i + 1];
         ds[3 * i + 2] = last;
       } else {
         ds[3 * i + 1] = last;
@@ -3383,6 +3434,8 @@ static int il_out(odis_ctx *ctx, Ops<T> &o) {
 }
 
 static int il_out_any(odis_ctx *ctx) {
+  const int rc = res_settle(ctx);
+  if (rc) return rc;
   return ctx->precision == ODIS_FP64 ? il_out(ctx, ctx->d) : il_out(ctx, ctx->f);
 }
 
@@ -3696,6 +3749,286 @@ static int read_kernel_times(odis_ctx *ctx) {
   return ODIS_OK;
 }
 
+// ---------------------------------------------------------------------------
+// resident launches (k_resident)
+// ---------------------------------------------------------------------------
+
+// Kernel variants: lanes and faces per lane.  The smallest that holds the
+// patches is taken (fewer lanes: cheaper barriers).
+struct ResVariant {
+  int lanes, faces;
+};
+constexpr ResVariant kResVariants[] = {{256, 1}, {512, 1}, {512, 3}, {1024, 1}, {1024, 2}};
+constexpr int kResVariantCount = 5;
+
+template <typename T, bool QUAD>
+static const void *res_kernel_q(int variant) {
+  switch (variant) {
+    case 0: return reinterpret_cast<const void *>(&k_resident<T, 256, 1, 1, QUAD>);
+    case 1: return reinterpret_cast<const void *>(&k_resident<T, 512, 1, 2, QUAD>);
+    case 2: return reinterpret_cast<const void *>(&k_resident<T, 512, 3, sizeof(T) == 4 ? 4 : 2, QUAD>);
+    case 3: return reinterpret_cast<const void *>(&k_resident<T, 1024, 1, 4, QUAD>);
+    default: return reinterpret_cast<const void *>(&k_resident<T, 1024, 2, 4, QUAD>);
+  }
+}
+template <typename T>
+static const void *res_kernel(const odis_ctx *ctx, int variant) {
+  return ctx->energy_quad || ctx->quad_drag ? res_kernel_q<T, true>(variant) : res_kernel_q<T, false>(variant);
+}
+
+constexpr int kResCells = 641;      // cells of a patch at most
+// fewer steps: a launch each.  A resident call costs about 30 us beside its
+// steps (loading the ocean, the arrival, the series kernel): 40 against 42 us
+// for 4 steps of 642 cells, 60 against 104 for 4 of 163842, FP64.
+constexpr int kResMinSteps = 4;
+constexpr size_t kResPartBytes = size_t(64) << 20;
+
+static bool res_wanted(const odis_ctx *ctx) {
+  return ctx->res_opt && !ctx->res.off && ctx->compact && ctx->one_kernel && ctx->patch == 64 &&
+         ctx->step_lanes == 4 && ctx->step_blocks == 0 && !ctx->use_graphs && ctx->il_opt != 1 &&
+         ctx->sh_mode == ODIS_SH_OFF;
+}
+
+// Time of a step of a resident round (us), from the sizes measured: FP64
+// 2.5 at 41 and 81 cells per patch, 3.1 at 161 to 321, 4.15 at 641; FP32 2.4
+// at 41, 2.8 at 641.  Nearly all of it is the exchange, so few rounds of
+// large patches beat many of small ones.
+static double res_round_us(double cells, bool fp64) { return 2.4 + (fp64 ? 2.7e-3 : 0.7e-3) * cells; }
+
+// Patches per instance for B instances on n_cu workgroups at once: the
+// number of rounds with the least total time, each round's instances
+// sharing the CUs evenly.  0: not even one instance fits.
+static int res_patches(int N, int B, int n_cu, bool fp64, int min_W) {
+  double best = 0.0;
+  int best_W = 0;
+  for (int rounds = 1; rounds <= B; rounds++) {
+    const int at_once = (B + rounds - 1) / rounds;
+    // no patch below 40 cells: it would be boundary only
+    const int W = std::min(n_cu / at_once, std::max(min_W, N / 40));
+    if (W < min_W) continue;
+    const double us = rounds * res_round_us(double(N) / W, fp64);
+    if (best_W == 0 || us < best) {
+      best = us;
+      best_W = W;
+    }
+  }
+  return best_W;
+}
+
+// Patches, variant and workspace for ctx->B instances; res.off when the
+// resident step cannot run (too large for the chip).
+template <typename T>
+static int res_setup(odis_ctx *ctx) {
+  ResDev &r = ctx->res;
+  if (r.W) return ODIS_OK;
+  const int N = ctx->N, E = ctx->E, B = ctx->B;
+  r.off = 1;
+  int dev = 0, n_cu = 0;
+  CK(hipGetDevice(&dev));
+  CK(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev));
+  // patches of at most kResCells cells; a partition that does not fit the
+  // largest variant (its boundary faces depend on the grid) is made finer
+  ResHost h;
+  int W = 0, v = 0, per_cu = 0;
+  int min_W = std::max(1, (N + kResCells - 1) / kResCells);
+  for (int tries = 0; tries < 4; tries++, min_W = W + std::max(1, W / 32)) {
+    W = ctx->res_opt > 1 ? ctx->res_opt : res_patches(N, B, n_cu, sizeof(T) == 8, min_W);
+    if (W < 1 || W > N / 16) return ODIS_OK;
+    if (!build_resident(N, E, ctx->cell_xyz, ctx->gi_host, ctx->cyc_host, W, h).empty()) return ODIS_OK;
+    for (v = 0; v < kResVariantCount; v++) {
+      const int lanes = kResVariants[v].lanes, cap = lanes * kResVariants[v].faces;
+      if (h.max_cells > lanes || h.max_face > cap || h.max_bnd > lanes) continue;
+      const size_t lds = res_lds_bytes<T>(lanes, h.max_cells, h.max_face, h.max_bnd, ctx->nfields);
+      if (lds > 160 * 1024) continue;
+      const void *k = res_kernel<T>(ctx, v);
+      if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)) != hipSuccess) {
+        (void)hipGetLastError();
+        continue;
+      }
+      CK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, lanes, lds));
+      if (per_cu > 0) break;
+    }
+    if (v < kResVariantCount || ctx->res_opt > 1) break;
+  }
+  if (v == kResVariantCount) return ODIS_OK;
+  const long long room = (long long)per_cu * n_cu;
+  if (room < W) return ODIS_OK;
+  const int at_once = int(std::min<long long>(B, room / W)), rounds = (B + at_once - 1) / at_once;
+  r.ipl = (B + rounds - 1) / rounds;  // even rounds
+  // the patch arrays in one buffer and one copy, then the workspaces
+  const int S = h.bptr[W];
+  std::vector<int> all;
+  auto put = [&](const std::vector<int> &x) {
+    const size_t at = all.size();
+    all.insert(all.end(), x.begin(), x.end());
+    return at;
+  };
+  const size_t o_cptr = put(h.cptr), o_fptr = put(h.fptr), o_bptr = put(h.bptr), o_cell = put(h.cell),
+               o_face = put(h.face), o_fcell = put(h.fcell), o_bface = put(h.bface), o_bcell = put(h.bcell),
+               o_bhalo = put(h.bhalo), o_bpeer = put(h.bpeer), o_cyc = all.size();
+  const size_t bytes = all.size() * sizeof(int) + h.cyc.size() * sizeof(unsigned short);
+  auto alloc = [&](void **dst, size_t n) -> int {
+    if (hipMalloc(dst, n) != hipSuccess) return fail(ctx, ODIS_E_NOMEM, "hipMalloc of the resident step");
+    r.allocs.push_back(*dst);
+    return ODIS_OK;
+  };
+  r.chunk = int(std::max<size_t>(size_t(kResMinSteps),
+                                 std::min<size_t>(size_t(std::min(ctx->chunk, 1024)),
+                                                  kResPartBytes / (sizeof(double) * size_t(B) * W))));
+  r.chunk = std::min(r.chunk, ctx->chunk);
+  void *ops = nullptr, *work = nullptr, *part = nullptr;
+  const size_t mail = size_t(r.ipl) * kResDepth * S * kResPlanes<T> * sizeof(uint4v);
+  int rc;
+  if ((rc = alloc(&ops, bytes)) || (rc = alloc(&work, 64 + mail)) ||
+      (rc = alloc(&part, size_t(B) * r.chunk * W * sizeof(double))))
+    return rc;
+  CK(hipMemcpy(ops, all.data(), all.size() * sizeof(int), hipMemcpyHostToDevice));
+  CK(hipMemcpy(static_cast<int *>(ops) + o_cyc, h.cyc.data(), h.cyc.size() * sizeof(unsigned short),
+               hipMemcpyHostToDevice));
+  CK(hipMemset(work, 0, 64 + mail));
+  if (!r.status) {
+    void *st = nullptr;
+    CK(hipHostMalloc(&st, 64, hipHostMallocDefault));
+    r.status = static_cast<unsigned *>(st);
+  }
+  *r.status = 0;
+  CK(hipDeviceSynchronize());
+  const int *base = static_cast<const int *>(ops);
+  r.cptr = base + o_cptr, r.fptr = base + o_fptr, r.bptr = base + o_bptr, r.cell = base + o_cell;
+  r.face = base + o_face, r.fcell = base + o_fcell, r.bface = base + o_bface, r.bcell = base + o_bcell;
+  r.bhalo = base + o_bhalo, r.bpeer = base + o_bpeer;
+  r.cyc = reinterpret_cast<const unsigned short *>(base + o_cyc);
+  r.ctl = static_cast<unsigned long long *>(work);
+  r.mail = reinterpret_cast<uint4v *>(static_cast<char *>(work) + 64);
+  r.part = static_cast<double *>(part);
+  r.W = W;
+  r.variant = v;
+  r.slots = S;
+  r.max_cells = h.max_cells;
+  r.max_face = h.max_face;
+  r.max_bnd = h.max_bnd;
+  r.off = 0;
+  return ODIS_OK;
+}
+
+// The last resident launch of each device: the next one, whatever its
+// context and stream, starts after it, so that two launches never hold a
+// part of the chip each.
+struct ResOrder {
+  std::mutex mu;
+  hipEvent_t ev = nullptr;
+  const odis_ctx *last = nullptr;
+};
+static ResOrder g_res_order[16];
+
+// Enqueue `count` steps of every instance from ctx->step in one launch.
+template <typename T>
+static int launch_resident(odis_ctx *ctx, Ops<T> &o, const double *table, int count) {
+  ResDev &r = ctx->res;
+  const int B = ctx->B, lanes = kResVariants[r.variant].lanes;
+  ResArgs<T> a;
+  a.E = ctx->E;
+  a.N = ctx->N;
+  a.B = B;
+  a.W = r.W;
+  a.ipl = r.ipl;
+  a.nfields = ctx->nfields;
+  a.energy_quad = ctx->energy_quad;
+  a.quad_drag = ctx->quad_drag;
+  a.count = count;
+  a.n0 = ctx->step;
+  a.seq0 = r.seq;
+  a.launch = ++r.launch;
+  const unsigned grid = unsigned(r.ipl) * unsigned(r.W);
+  r.arrived += grid;
+  a.arrive = r.arrived;
+  a.g_coef = o.g_coef;
+  a.fcor = o.fcor;
+  a.farea = o.farea;
+  a.fdist = o.fdist;
+  a.flen = o.flen;
+  a.kite = o.kite;
+  a.area = o.area;
+  a.cellS = o.cellS;
+  a.info = o.info;
+  a.inst = ctx->inst;
+  a.table = table;
+  a.cptr = r.cptr;
+  a.fptr = r.fptr;
+  a.bptr = r.bptr;
+  a.cell = r.cell;
+  a.face = r.face;
+  a.fcell = r.fcell;
+  a.bface = r.bface;
+  a.bcell = r.bcell;
+  a.bhalo = r.bhalo;
+  a.bpeer = r.bpeer;
+  a.cyc = r.cyc;
+  a.max_cells = r.max_cells;
+  a.max_face = r.max_face;
+  a.max_bnd = r.max_bnd;
+  a.v = o.v[ctx->cur];
+  a.eta = o.eta[ctx->cur];
+  a.ts = o.ts[ctx->cur];
+  a.v_out = o.v[ctx->cur ^ 1];
+  a.eta_out = o.eta[ctx->cur ^ 1];
+  a.ts_out = o.ts[ctx->cur ^ 1];
+  a.ring_v = o.ring_v;
+  a.ring_e = o.ring_e;
+  a.part = r.part;
+  a.mail = r.mail;
+  a.slots = r.slots;
+  a.ctl = r.ctl;
+  a.status = r.status;
+  r.seq += unsigned(count) * unsigned((B + r.ipl - 1) / r.ipl);
+  const size_t lds = res_lds_bytes<T>(lanes, r.max_cells, r.max_face, r.max_bnd, ctx->nfields);
+  int dev = 0;
+  CK(hipGetDevice(&dev));
+  ResOrder &ord = g_res_order[dev & 15];
+  {
+    std::lock_guard<std::mutex> lock(ord.mu);
+    if (!ord.ev) CK(hipEventCreateWithFlags(&ord.ev, hipEventDisableTiming));
+    if (ord.last && ord.last != ctx) CK(hipStreamWaitEvent(ctx->stream, ord.ev, 0));
+    void *params[] = {&a};
+    CK(hipLaunchKernel(res_kernel<T>(ctx, r.variant), dim3(grid), dim3(lanes), params, lds, ctx->stream));
+    CK(hipEventRecord(ord.ev, ctx->stream));
+    ord.last = ctx;
+  }
+  r.pending.push_back({a.launch, ctx->step, ctx->cur});
+  hipLaunchKernelGGL(k_resident_series, dim3(count, B), dim3(64), 0, ctx->stream, r.part, r.W, count, ctx->step,
+                     ctx->dconst, ctx->series, ctx->nonfinite, ctx->cap);
+  CK(hipGetLastError());
+  ctx->cur ^= 1;
+  return ODIS_OK;
+}
+
+template <typename T>
+static int step_t(odis_ctx *ctx, Ops<T> &o, int n_steps);
+
+// Wait for the resident launches enqueued so far and learn whether they ran.
+// Steps of a launch that was taken back (nothing of it, nor of the later
+// ones, was written) are stepped again with a launch each.  Called before
+// anything reads the state or steps by another kernel.
+static int res_settle(odis_ctx *ctx) {
+  ResDev &r = ctx->res;
+  if (r.pending.empty()) return ODIS_OK;
+  CK(hipStreamSynchronize(ctx->stream));
+  const std::vector<ResDev::Pending> sent = std::move(r.pending);
+  r.pending.clear();
+  const unsigned st = *static_cast<volatile unsigned *>(r.status);
+  if (st == 0) return ODIS_OK;
+  r.off = 1;
+  if (st == kResFailed) return fail(ctx, ODIS_E_HIP, "resident step: a workgroup did not answer in time");
+  for (const auto &p : sent)
+    if (p.launch == st) {
+      const long long n = ctx->step - p.n0;
+      ctx->step = p.n0;
+      ctx->cur = p.cur;
+      return ctx->precision == ODIS_FP64 ? step_t(ctx, ctx->d, int(n)) : step_t(ctx, ctx->f, int(n));
+    }
+  return fail(ctx, ODIS_E_HIP, "resident step: unknown launch taken back");
+}
+
 template <typename T>
 static int step_t(odis_ctx *ctx, Ops<T> &o, int n_steps) {
   // Timing mode (ctx->timing = T > 0): the kernels of every T-th step get
@@ -3707,26 +4040,58 @@ static int step_t(odis_ctx *ctx, Ops<T> &o, int n_steps) {
   std::vector<ChunkEvents> sampled;
   size_t ev_used = 0;
   int done = 0;
-  const bool il = il_wanted(ctx);
-  if (il) {
-    if (!ctx->il_fresh) {  // the instance-major arrays are current: copy them in
-      if ((rc = ensure_ts(ctx, o)) || (rc = il_alloc<T>(ctx)) || (rc = il_convert(ctx, o, true))) return rc;
-      ctx->il_fresh = 1;
+  // the state in the layout of the step launches of the next stretch
+  auto enter = [&](bool il) -> int {
+    if (il) {
+      if (!ctx->il_fresh) {  // the instance-major arrays are current: copy them in
+        int e;
+        if ((e = ensure_ts(ctx, o)) || (e = il_alloc<T>(ctx)) || (e = il_convert(ctx, o, true))) return e;
+        ctx->il_fresh = 1;
+      }
+      const int e = il_records(ctx, o);
+      if (e) return e;
+      ctx->std_fresh = 0;
+    } else {
+      int e;
+      if ((e = il_out(ctx, o)) || (e = ensure_ts(ctx, o))) return e;
+      ctx->il_fresh = 0;
     }
-    if ((rc = il_records(ctx, o))) return rc;
-    ctx->std_fresh = 0;
-  } else {
-    if ((rc = il_out(ctx, o)) || (rc = ensure_ts(ctx, o))) return rc;
-    ctx->il_fresh = 0;
-  }
+    return ODIS_OK;
+  };
+  if (res_wanted(ctx) && n_steps >= kResMinSteps && (rc = res_setup<T>(ctx))) return rc;
+  const bool resident = res_wanted(ctx) && n_steps >= kResMinSteps;
+  if (!resident && ((rc = res_settle(ctx)) || (rc = enter(il_wanted(ctx))))) return rc;
   while (done < n_steps) {
     if (ctx->stop_flag) {
       ctx->stop_flag = 0;
       return fail(ctx, ODIS_E_STOPPED, "stop requested");
     }
     const int left = n_steps - done;
+    if (resident) {
+      // up to the next sampled step, which is launched by itself
+      const long long T_s = ctx->timing, ahead = T_s > 0 ? (T_s - ctx->step % T_s) % T_s : left;
+      int run = int(std::min<long long>(left, ahead));
+      if (run > ctx->res.chunk) {  // near-equal launches, none too short to be one
+        const int parts = (run + ctx->res.chunk - 1) / ctx->res.chunk;
+        run = (run + parts - 1) / parts;
+      }
+      if (run >= kResMinSteps) {
+        if ((rc = enter(false))) return rc;
+        const double *table = nullptr;
+        if ((rc = stage_coefficients(ctx, ctx->step, run, &table))) return rc;
+        if ((rc = launch_resident(ctx, o, table, run))) return rc;
+        ctx->step += run;
+        done += run;
+        continue;
+      }
+      if ((rc = res_settle(ctx)) || (rc = enter(il_wanted(ctx)))) return rc;
+    }
     const bool graph_fits = ctx->use_graphs && left >= ctx->graph_steps;
-    const int count = graph_fits ? ctx->graph_steps : std::min(ctx->chunk, left);
+    int count = graph_fits ? ctx->graph_steps : std::min(ctx->chunk, left);
+    if (resident && ctx->timing > 0) {  // this step if it is sampled, else those up to the next sampled one
+      const long long T_s = ctx->timing, ahead = (T_s - ctx->step % T_s) % T_s;
+      count = std::min<int>(count, std::max<int>(1, int(std::min<long long>(ahead, count))));
+    }
     // does [step, step + count) hold a multiple of the timing stride?
     const bool sample = ctx->timing > 0 && ((ctx->step + ctx->timing - 1) / ctx->timing) * ctx->timing <
                                                ctx->step + count;
@@ -3760,7 +4125,10 @@ static int step_impl(odis_ctx *ctx, int n_steps, int flags) {
   if (n_steps < 0) return fail(ctx, ODIS_E_INVALID, "n_steps < 0");
   int rc = ctx->precision == ODIS_FP64 ? step_t(ctx, ctx->d, n_steps) : step_t(ctx, ctx->f, n_steps);
   if (rc) return rc;
-  if (flags & ODIS_SYNC) CK(hipStreamSynchronize(ctx->stream));
+  if (flags & ODIS_SYNC) {
+    if ((rc = res_settle(ctx))) return rc;
+    CK(hipStreamSynchronize(ctx->stream));
+  }
   return ODIS_OK;
 }
 
@@ -3770,13 +4138,15 @@ extern "C" int odis_step(odis_ctx *ctx, int n_steps, int flags) {
 
 extern "C" int odis_sync(odis_ctx *ctx) {
   if (!ctx) return ODIS_E_INVALID;
+  const int rc = guarded(ctx, [&] { return res_settle(ctx); });
+  if (rc) return rc;
   CK(hipStreamSynchronize(ctx->stream));
   return ODIS_OK;
 }
 
 template <typename T>
 static int diss_t(odis_ctx *ctx, Ops<T> &o) {
-  int rc = il_out(ctx, o);
+  int rc = il_out_any(ctx);
   if (rc || (rc = ensure_ts(ctx, o))) return rc;
   FaceArgs<T> fa = face_args(ctx, o);
   const dim3 gf(ctx->nb_face, ctx->B), blk(kBlock);
@@ -3812,6 +4182,8 @@ extern "C" int odis_series_capacity(const odis_ctx *ctx) { return ctx ? ctx->cap
 static int get_dissipation_series_impl(odis_ctx *ctx, int inst, long long first, int count, double *out) {
   if (!ctx || !out || count < 0) return ODIS_E_INVALID;
   if (inst < 0 || inst >= ctx->B) return fail(ctx, ODIS_E_RANGE, "instance out of range");
+  const int rc = res_settle(ctx);
+  if (rc) return rc;
   CK(hipStreamSynchronize(ctx->stream));
   // series[k] exists for max(series_lo, step - cap) <= k < step
   if (first < ctx->series_lo || first + count > ctx->step || first < ctx->step - ctx->cap)
@@ -3881,7 +4253,7 @@ template <typename T>
 static int orbit_stats_t(odis_ctx *ctx, Ops<T> &o, int n, const int *inst, const int *ns, double *out) {
   const int B = ctx->B;
   const long long E = ctx->E, N = ctx->N;
-  int rc = il_out(ctx, o);
+  int rc = il_out_any(ctx);
   if (rc) return rc;
   if (!ctx->snap) {
     if ((rc = dev_alloc(ctx, &ctx->snap, size_t(B) * size_t(E + N)))) return rc;
@@ -3942,7 +4314,7 @@ static int compact_slots(odis_ctx *ctx, U *base, size_t per, const int *keep, in
 template <typename T>
 static int retire_t(odis_ctx *ctx, Ops<T> &o, const int *keep, int n_keep) {
   const size_t E = ctx->E, N = ctx->N;
-  int rc = il_out(ctx, o);  // the instance-major arrays hold the state
+  int rc = il_out_any(ctx);  // the instance-major arrays hold the state
   if (rc) return rc;
   for (int k = 0; k < 2 && !rc; k++) {
     if (!rc) rc = compact_slots(ctx, o.v[k], E, keep, n_keep);
@@ -3962,6 +4334,12 @@ static int retire_t(odis_ctx *ctx, Ops<T> &o, const int *keep, int n_keep) {
     for (int j = 0; j < n_keep; j++) vec[j] = vec[keep[j]];
     vec.resize(n_keep);
   };
+  {  // the resident step is set up again for the kept instances
+    const int off = ctx->res.off;
+    CK(hipStreamSynchronize(ctx->stream));
+    res_free(ctx);
+    ctx->res.off = off;
+  }
   pick(ctx->params);
   pick(ctx->tides);
   pick(ctx->init_hist_v);
@@ -4000,7 +4378,7 @@ extern "C" int odis_retire(odis_ctx *ctx, const int *keep, int n_keep) {
 template <typename T>
 static int vel_t(odis_ctx *ctx, Ops<T> &o, int b, const double *normal, double *uv) {
   const int E = ctx->E;
-  const int rc = il_out(ctx, o);
+  const int rc = il_out_any(ctx);
   if (rc) return rc;
   std::vector<double> nd(size_t(2) * E);
   for (int r = 0; r < E; r++) {
@@ -4062,6 +4440,17 @@ extern "C" int odis_enable_timing(odis_ctx *ctx, int stride) {
 
 static int set_option_impl(odis_ctx *ctx, int option, int value) {
   if (!ctx) return ODIS_E_INVALID;
+  const int settled = res_settle(ctx);
+  if (settled) return settled;
+  if (option == ODIS_OPT_RESIDENT) {
+    if (value < 0) return fail(ctx, ODIS_E_INVALID, "resident steps: 0 (off), 1 (automatic) or the patches per instance");
+    if (value != ctx->res_opt) {
+      CK(hipStreamSynchronize(ctx->stream));
+      res_free(ctx);
+      ctx->res_opt = value;
+    }
+    return ODIS_OK;
+  }
   if (option == ODIS_OPT_GRAPHS) {
     ctx->use_graphs = value ? 1 : 0;
     return ODIS_OK;
@@ -4178,6 +4567,7 @@ extern "C" int odis_get_option(odis_ctx *ctx, int option, int *value) {
   else if (option == ODIS_OPT_IL_UNROLL) *value = ctx->il_unroll;
   else if (option == ODIS_OPT_IL_ORDER) *value = ctx->il_order;
   else if (option == ODIS_OPT_IL_RECORDS) *value = ctx->il_rec;
+  else if (option == ODIS_OPT_RESIDENT) *value = ctx->res_opt;
   else return fail(ctx, ODIS_E_INVALID, "unknown option");
   return ODIS_OK;
 }
@@ -4418,6 +4808,8 @@ static int sh_set_basis_impl(odis_ctx *ctx, int l_max, const double *beta, int m
   if (mode != ODIS_SH_OFF && mode != ODIS_SH_FP64 && mode != ODIS_SH_SPLIT_BF16 && mode != ODIS_SH_RECUR &&
       mode != ODIS_SH_MFMA)
     return fail(ctx, ODIS_E_INVALID, "bad sh mode");
+  const int settled = res_settle(ctx);
+  if (settled) return settled;
   CK(hipStreamSynchronize(ctx->stream));
   drop_graphs(ctx);
   for (void *p : ctx->sh_allocs) (void)hipFree(p);

@@ -311,7 +311,15 @@ int odis_request_stop(odis_ctx *ctx);
  *                    per-face and per-cell records that each group of 16
  *                    lanes loads once and shares by row broadcasts (tides
  *                    with at most 4 forcing fields), 0 every lane loads
- *                    every operand.  Same state bit for bit. */
+ *                    every operand.  Same state bit for bit.
+ *  ODIS_OPT_RESIDENT many steps per launch, the ocean held in registers and
+ *                    LDS of one workgroup per patch: 1 (default) when the
+ *                    ocean fits the chip, no SH basis is set, the launch
+ *                    options above are at their defaults (interleaving 0 or
+ *                    2) and an odis_step call has enough steps; 0 off; a
+ *                    larger value: that many patches per instance.  Steps
+ *                    sampled for timing are launched by themselves.  Same
+ *                    state bit for bit; dissipation sums differ by rounding. */
 #define ODIS_OPT_GRAPHS     1
 #define ODIS_OPT_COMPACT    2
 #define ODIS_OPT_ONE_KERNEL 3
@@ -324,6 +332,7 @@ int odis_request_stop(odis_ctx *ctx);
 #define ODIS_OPT_IL_UNROLL 10
 #define ODIS_OPT_IL_ORDER 11
 #define ODIS_OPT_IL_RECORDS 12
+#define ODIS_OPT_RESIDENT 13
 int odis_set_option(odis_ctx *ctx, int option, int value);
 int odis_get_option(odis_ctx *ctx, int option, int *value);
 /* Timing for benchmarks: with stride T > 0, the kernels of every step n of
