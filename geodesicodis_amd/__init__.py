@@ -393,8 +393,8 @@ class Context:
 
     def get_state(self, inst=0):
         m = self.mesh
-        v, dv = np.zeros(m.E), np.zeros(m.E * 3)
-        eta, de = np.zeros(m.N), np.zeros(m.N * 3)
+        v, dv = np.empty(m.E), np.empty(m.E * 3)
+        eta, de = np.empty(m.N), np.empty(m.N * 3)
         it = ctypes.c_longlong()
         self._check(lib().odis_get_state(self._h, int(inst), _dp(v), _dp(dv), _dp(eta), _dp(de),
                                          ctypes.byref(it)))
@@ -438,7 +438,7 @@ class Context:
 
     def velocity_en(self, inst=0):
         normal = np.ascontiguousarray(self.mesh.get("face_normal"))
-        uv = np.zeros(self.mesh.E * 2)
+        uv = np.empty(self.mesh.E * 2)
         self._check(lib().odis_get_velocity_en(self._h, int(inst), _dp(normal), _dp(uv)))
         return uv.reshape(-1, 2)
 
@@ -470,7 +470,7 @@ class Context:
 
     def velocity_xyz(self, inst=0):
         """Cartesian velocity [N, 3] at cell centres (reference numbering)."""
-        out = np.zeros(self.mesh.N * 3)
+        out = np.empty(self.mesh.N * 3)
         self._check(lib().odis_velocity_xyz(self._h, int(inst), _dp(out)))
         return out.reshape(-1, 3)
 

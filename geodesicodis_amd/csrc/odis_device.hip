@@ -873,43 +873,92 @@ __global__ __launch_bounds__(kBlock) void k_diss_final(const double *partials, i
   if (threadIdx.x == 0) out[b] = t * dconst[b];
 }
 
-// (east, north) velocity per face: n v_n + t v_t with t = (n_y, -n_x)
-// (src/interpolation.cpp:49-58).
+// State and output kernels write reference order straight into pinned host
+// memory, consecutive lanes to consecutive doubles, at the rate of a DMA copy
+// (54 GB/s); the host has nothing left to permute.  A full FP64 state of
+// 163842 cells (16 MB): 0.7 ms, 2.7 with pageable copies and host loops; of
+// 642 cells: 17 us, 60.
+//
+// One state to the host: v[E], dvdt[E][3], eta[N], detadt[N][3] as asked for,
+// one after the other; a history row is (slot q0, q1, q2) of the ring, 0 where
+// a slot is negative.  out: the doubles [first, first + count) of that.
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_velocity_en(int E, const int *tri_idx, const T *tri_coef,
-                                                        const T *v, const double *normal, double *uv) {
-  const int e = blockIdx.x * kBlock + threadIdx.x;
-  if (e >= E) return;
+struct StateOut {
+  const T *x;                // v or eta; null: not asked for
+  const T *ring;             // its history ring; null: not asked for
+  const int *perm;           // reference -> device
+  int n;
+  int q[3];
+};
+template <typename T>
+__device__ __forceinline__ bool state_out(const StateOut<T> &a, long long &t, double &value) {
+  if (a.x) {
+    if (t < a.n) {
+      value = double(a.x[a.perm[t]]);
+      return true;
+    }
+    t -= a.n;
+  }
+  if (a.ring) {
+    if (t < 3LL * a.n) {
+      const int i = int(t / 3), s = a.q[t - 3LL * i];
+      value = s < 0 ? 0.0 : double(a.ring[size_t(s) * a.n + a.perm[i]]);
+      return true;
+    }
+    t -= 3LL * a.n;
+  }
+  return false;
+}
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_state_out(StateOut<T> faces, StateOut<T> cells, long long first, int count,
+                                                      double *out) {
+  const int k = blockIdx.x * kBlock + threadIdx.x;
+  if (k >= count) return;
+  long long t = first + k;
+  double value = 0.0;
+  if (!state_out(faces, t, value)) state_out(cells, t, value);
+  out[k] = value;
+}
+
+// (east, north) velocity per face: n v_n + t v_t with t = (n_y, -n_x)
+// (src/interpolation.cpp:49-58).  normal and uv: of the reference faces
+// [first, first + count).
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_velocity_en(int E, int first, int count, const int *__restrict__ perm,
+                                                        const int *tri_idx, const T *tri_coef, const T *v,
+                                                        const double2 *normal, double2 *uv) {
+  const int i = blockIdx.x * kBlock + threadIdx.x;
+  if (i >= count) return;
+  const int e = perm[first + i];
   double vt = 0.0;
   for (int j = 0; j < 10; ++j) vt += double(tri_coef[j * E + e]) * double(v[tri_idx[j * E + e]]);
-  const double nx = normal[2 * e], ny = normal[2 * e + 1], vn = double(v[e]);
-  uv[2 * e] = nx * vn + ny * vt;
-  uv[2 * e + 1] = ny * vn + (-nx) * vt;
+  const double2 n = normal[i];
+  const double vn = double(v[e]);
+  uv[i] = make_double2(n.x * vn + n.y * vt, n.y * vn + (-n.x) * vt);
 }
 
 // RBF reconstruction of the Cartesian velocity at cell centres
 // (interpolateVelocityCartRBF, src/interpolation.cpp:64-174): per device
 // cell the reference operator's 3 x k block (k <= 6 faces, slot-major, the
-// CSR's column order), out [3][N].
+// CSR's column order); out: the doubles [first, first + count) of xyz[N][3] in
+// reference order, one lane each.
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_velocity_xyz(int N, const int *__restrict__ idx,
+__global__ __launch_bounds__(kBlock) void k_velocity_xyz(int N, int first, int count, const int *__restrict__ perm,
+                                                         const int *__restrict__ idx,
                                                          const double *__restrict__ w, const T *__restrict__ v,
                                                          double *out) {
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= N) return;
-  double u[6];
+  const int k = blockIdx.x * kBlock + threadIdx.x;
+  if (k >= count) return;
+  const int t = first + k;
+  const int c = t % 3, i = perm[t / 3];
+  double acc = 0.0;
 #pragma unroll
   for (int j = 0; j < 6; ++j) {
     const int f = idx[j * N + i];
-    u[j] = f >= 0 ? double(v[f]) : 0.0;
+    const double u = f >= 0 ? double(v[f]) : 0.0;
+    acc += w[(c * 6 + j) * N + i] * u;
   }
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    double acc = 0.0;
-#pragma unroll
-    for (int j = 0; j < 6; ++j) acc += w[(c * 6 + j) * N + i] * u[j];
-    out[c * N + i] = acc;
-  }
+  out[k] = acc;
 }
 
 // CSR rows of the lat-lon interpolation: one wavefront per row, the eta
@@ -2120,7 +2169,7 @@ struct ResDev {
   unsigned long long *ctl = nullptr;
   double *part = nullptr;
   int chunk = 0;               // steps per launch at most
-  unsigned *status = nullptr;  // pinned host memory
+  unsigned *status = nullptr;  // pinned host memory, behind the context's first coefficient table
   unsigned seq = 0, launch = 0;
   unsigned long long arrived = 0;
   int off = 0;                 // not usable on this context (or taken back once)
@@ -2148,6 +2197,7 @@ struct odis_ctx {
   int energy_quad = 0, quad_drag = 0;
   hipStream_t stream = nullptr;
   std::vector<int> cell_perm, cell_inv, face_perm, face_inv;  // ref -> dev, dev -> ref
+  int *cell_perm_dev = nullptr, *face_perm_dev = nullptr;     // the first of each on the device
   Ops<double> d;
   Ops<float> f;
   int cur = 0;                 // v is v[cur] between calls
@@ -2196,6 +2246,7 @@ struct odis_ctx {
   int chunk = 0;
   double *coef_dev[2] = {nullptr, nullptr};
   double *coef_host[2] = {nullptr, nullptr};
+  size_t coef_doubles = 0;     // of a table; the host buffers hold 8 more
   hipEvent_t coef_ev[2] = {nullptr, nullptr};
   int coef_next = 0, coef_last = 0;
   // graphs of graph_steps steps, one per (coefficient buffer, v parity)
@@ -2234,9 +2285,9 @@ struct odis_ctx {
   double *ll_val = nullptr, *ll_out = nullptr;
   std::vector<void *> ll_allocs;
   // RBF Cartesian velocity operator: [6][N] device face ids (-1 pad),
-  // [3][6][N] coefficients, [3][N] output
+  // [3][6][N] coefficients
   int *rbf_idx = nullptr;
-  double *rbf_w = nullptr, *rbf_out = nullptr;
+  double *rbf_w = nullptr;
   std::vector<void *> rbf_allocs;
   std::string err;
 };
@@ -2292,6 +2343,118 @@ static int upload(odis_ctx *ctx, T **p, const std::vector<T> &h) {
   int rc = dev_alloc(ctx, p, h.size());
   if (rc) return rc;
   CK(hipMemcpy(*p, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice));
+  return ODIS_OK;
+}
+
+// Pinned host buffers of the state and output calls, shared by the process's
+// contexts: a call takes one and gives it back when it returns (its kernels
+// have finished by then), so there are as many as calls at one time.  At most
+// kStageKeep are kept for later calls, and none once the last context is
+// destroyed.  Small on purpose: the GPU's first accesses to pinned pages after
+// the page tables changed are slow (a 21 MB buffer cost the first call on a
+// new context 10 ms), so a large output goes through the same few pages.
+constexpr size_t kStageDoubles = size_t(1) << 18;  // 2 MB
+constexpr size_t kStageKeep = 4;
+struct StagePool {
+  std::mutex mu;
+  double *kept[kStageKeep] = {};
+  int contexts = 0;
+
+  void context_made() {
+    std::lock_guard<std::mutex> lock(mu);
+    contexts++;
+  }
+  void context_gone() {
+    std::lock_guard<std::mutex> lock(mu);
+    if (--contexts > 0) return;
+    for (double *&p : kept) {
+      if (p) (void)hipHostFree(p);
+      p = nullptr;
+    }
+  }
+};
+static StagePool g_stage_pool;
+// One buffer for the length of a call; p is null when none could be had.
+struct Stage {
+  double *p = nullptr;
+  Stage() {
+    {
+      std::lock_guard<std::mutex> lock(g_stage_pool.mu);
+      for (double *&q : g_stage_pool.kept)
+        if (q) {
+          std::swap(p, q);
+          return;
+        }
+    }
+    void *q = nullptr;
+    if (hipHostMalloc(&q, kStageDoubles * sizeof(double), hipHostMallocDefault) == hipSuccess)
+      p = static_cast<double *>(q);
+    else
+      (void)hipGetLastError();
+  }
+  ~Stage() {
+    if (!p) return;
+    std::lock_guard<std::mutex> lock(g_stage_pool.mu);
+    if (g_stage_pool.contexts > 0)
+      for (double *&q : g_stage_pool.kept)
+        if (!q) {
+          q = p;
+          return;
+        }
+    (void)hipHostFree(p);
+  }
+  Stage(const Stage &) = delete;
+  Stage &operator=(const Stage &) = delete;
+};
+
+// Runs `items` pieces of `per` doubles of pinned memory each through a Stage:
+// fill(first, count, buf) puts the caller's input there, launch(first, count,
+// buf) enqueues the kernel of those items on ctx->stream, take(first, count,
+// buf) copies the result to the caller.  More than a buffer's worth goes in
+// quarter buffers, up to four kernels ahead of the copies, so that kernels
+// and PCIe run beside them.  (Four threads copying took 2.6 instead of 2.8 ms
+// for 500 steps and a state of 163842 cells into warm memory, but 1.9 instead of 0.9
+// ms for 5.2 MB into memory the caller has just got: page faults of several
+// threads hold each other up.)
+template <typename Fill, typename Launch, typename Take>
+static int staged(odis_ctx *ctx, size_t items, size_t per, Fill fill, Launch launch, Take take) {
+  if (!items) return ODIS_OK;
+  Stage stage;
+  if (!stage.p) return fail(ctx, ODIS_E_NOMEM, "hipHostMalloc of the output buffer");
+  if (items * per <= kStageDoubles) {
+    fill(size_t(0), items, stage.p);
+    launch(size_t(0), items, stage.p);
+    CK(hipGetLastError());
+    CK(hipStreamSynchronize(ctx->stream));
+    take(size_t(0), items, stage.p);
+    return ODIS_OK;
+  }
+  constexpr size_t kSlots = 4;
+  const size_t part = kStageDoubles / kSlots / per, n_part = (items + part - 1) / part;
+  hipEvent_t done[kSlots] = {};
+  hipError_t e = hipSuccess;
+  for (hipEvent_t &d : done)
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&d, hipEventDisableTiming);
+  auto buf = [&](size_t c) { return stage.p + c % kSlots * (kStageDoubles / kSlots); };
+  auto count = [&](size_t c) { return std::min(part, items - c * part); };
+  auto send = [&](size_t c) {
+    if (c >= n_part || e != hipSuccess) return;
+    fill(c * part, count(c), buf(c));
+    launch(c * part, count(c), buf(c));
+    e = hipGetLastError();
+    if (e == hipSuccess) e = hipEventRecord(done[c % kSlots], ctx->stream);
+  };
+  for (size_t c = 0; c < kSlots; c++) send(c);
+  for (size_t c = 0; c < n_part && e == hipSuccess; c++) {
+    e = hipEventSynchronize(done[c % kSlots]);
+    if (e == hipSuccess) take(c * part, count(c), buf(c));
+    send(c + kSlots);
+  }
+  const hipError_t drained = hipStreamSynchronize(ctx->stream);  // nothing still writes the buffer
+  for (hipEvent_t d : done)
+    if (d) (void)hipEventDestroy(d);
+  CK(e);
+  CK(drained);
   return ODIS_OK;
 }
 
@@ -2501,7 +2664,6 @@ static bool res_wanted(const odis_ctx *ctx);
 
 static void res_free(odis_ctx *ctx) {
   for (void *p : ctx->res.allocs) (void)hipFree(p);
-  if (ctx->res.status) (void)hipHostFree(ctx->res.status);
   ctx->res = ResDev();
 }
 
@@ -2517,6 +2679,7 @@ extern "C" int odis_destroy(odis_ctx *ctx) {
     if (ctx->coef_host[k]) (void)hipHostFree(ctx->coef_host[k]);
   }
   res_free(ctx);
+  g_stage_pool.context_gone();
   for (void *p : ctx->allocs) (void)hipFree(p);
   for (void *p : ctx->rbf_allocs) (void)hipFree(p);
   for (void *p : ctx->ll_allocs) (void)hipFree(p);
@@ -2565,6 +2728,7 @@ static int create_impl(const odis_mesh_desc *m, const odis_params *params, int n
 
   odis_ctx *ctx = new odis_ctx();
   *building = ctx;
+  g_stage_pool.context_made();
   ctx->N = N;
   ctx->E = E;
   ctx->B = n_inst;
@@ -2748,6 +2912,12 @@ static int create_impl(const odis_mesh_desc *m, const odis_params *params, int n
     ctx->tides[b] = make_tide(p);
     ctx->tides[b].nfields = K;
   }
+  if (!rc) {
+    std::vector<int> perm(ctx->face_perm);
+    perm.insert(perm.end(), ctx->cell_perm.begin(), ctx->cell_perm.end());
+    rc = upload(ctx, &ctx->face_perm_dev, perm);
+    ctx->cell_perm_dev = ctx->face_perm_dev + E;
+  }
   if (!rc) rc = upload(ctx, &ctx->inst, inst);
   if (!rc) rc = upload(ctx, &ctx->dconst, dconst);
   ctx->part_cap = std::max(ctx->nb_face, (N + 63) / 64);
@@ -2760,10 +2930,12 @@ static int create_impl(const odis_mesh_desc *m, const odis_params *params, int n
   ctx->chunk &= ~1;
   ctx->graph_steps = std::min(64, ctx->chunk);
   const size_t tab = 8 + size_t(ctx->chunk) * n_inst * 8;
+  ctx->coef_doubles = tab;
   for (int k = 0; k < 2 && !rc; k++) {
     rc = dev_alloc(ctx, &ctx->coef_dev[k], tab);
     if (!rc) {
-      he = hipHostMalloc(reinterpret_cast<void **>(&ctx->coef_host[k]), tab * sizeof(double), hipHostMallocDefault);
+      he = hipHostMalloc(reinterpret_cast<void **>(&ctx->coef_host[k]), (tab + 8) * sizeof(double),
+                         hipHostMallocDefault);
       if (he == hipSuccess) he = hipEventCreateWithFlags(&ctx->coef_ev[k], hipEventDisableTiming);
       if (he == hipSuccess) he = hipEventRecord(ctx->coef_ev[k], ctx->stream);
       if (he != hipSuccess) rc = fail(ctx, ODIS_E_HIP, std::string("coef table: ") + hipGetErrorString(he));
@@ -2877,44 +3049,62 @@ extern "C" int odis_set_state(odis_ctx *ctx, int inst, const double *v, const do
 template <typename T>
 static int get_state_t(odis_ctx *ctx, Ops<T> &o, int b, double *v, double *dv, double *eta, double *de,
                        long long k) {
-  const int E = ctx->E, N = ctx->N;
-  const bool load = ctx->params[b].init_load != 0;
-  const size_t bE = size_t(b) * E, bN = size_t(b) * N;
-  if (v) {
-    std::vector<T> h(E);
-    CK(hipMemcpy(h.data(), o.v[ctx->cur] + bE, E * sizeof(T), hipMemcpyDeviceToHost));
-    for (int r = 0; r < E; r++) v[ctx->face_inv[r]] = double(h[r]);
+  const size_t E = ctx->E, N = ctx->N;
+  const bool euler = k == 1 && ctx->params[b].init_load == 0;  // the row's middle entry is as it was set
+  StateOut<T> f{}, c{};
+  f.n = int(E), f.perm = ctx->face_perm_dev;
+  c.n = int(N), c.perm = ctx->cell_perm_dev;
+  for (StateOut<T> *a : {&f, &c}) {
+    a->q[0] = int((k + 2) % 3);  // of step k - 1
+    a->q[1] = euler ? -1 : a->q[0];
+    a->q[2] = euler ? a->q[0] : int((k + 1) % 3);
   }
-  if (eta) {
-    std::vector<T> h(N);
-    CK(hipMemcpy(h.data(), o.eta[ctx->cur] + bN, N * sizeof(T), hipMemcpyDeviceToHost));
-    for (int r = 0; r < N; r++) eta[ctx->cell_inv[r]] = double(h[r]);
-  }
-  auto get_hist = [&](T *ring, int M, const std::vector<int> &inv, double *ds,
-                      const std::vector<double> &keep) -> int {
-    std::vector<T> all(size_t(3) * M);
-    CK(hipMemcpy(all.data(), ring + size_t(b) * 3 * M, all.size() * sizeof(T), hipMemcpyDeviceToHost));
-    for (int r = 0; r < M; r++) {
-      const int i = inv[r];
-      if (k == 0) {  // no step since set_state: the history as set
-        for (int q = 0; q < 3; q++) ds[3 * i + q] = keep.empty() ? 0.0 : keep[3 * i + q];
-        continue;
-      }
-      const double last = double(all[size_t((k - 1) % 3) * M + r]);
-      ds[3 * i + 0] = last;
-      if (k == 1 && !load) {
-        ds[3 * i + 1] = keep.empty() ? 0.0 : keep[3 * i + 1];
-        ds[3 * i + 2] = last;
-      } else {
-        ds[3 * i + 1] = last;
-        ds[3 * i + 2] = double(all[size_t((k + 1) % 3) * M + r]);
-      }
-    }
-    return ODIS_OK;
+  if (v) f.x = o.v[ctx->cur] + b * E;
+  if (eta) c.x = o.eta[ctx->cur] + b * N;
+  if (dv && k > 0) f.ring = o.ring_v + b * 3 * E;
+  if (de && k > 0) c.ring = o.ring_e + b * 3 * N;
+  const size_t n_out = (f.x ? E : 0) + (f.ring ? 3 * E : 0) + (c.x ? N : 0) + (c.ring ? 3 * N : 0);
+  // where the doubles [lo, lo + n) of the output go
+  struct Seg {
+    double *dst;
+    size_t lo, n;
+  } seg[4];
+  int n_seg = 0;
+  size_t at = 0;
+  auto add = [&](bool on, double *dst, size_t n) {
+    if (!on) return;
+    seg[n_seg++] = {dst, at, n};
+    at += n;
   };
-  int rc;
-  if (dv && (rc = get_hist(o.ring_v, E, ctx->face_inv, dv, ctx->init_hist_v[b]))) return rc;
-  if (de && (rc = get_hist(o.ring_e, N, ctx->cell_inv, de, ctx->init_hist_e[b]))) return rc;
+  add(f.x, v, E);
+  add(f.ring, dv, 3 * E);
+  add(c.x, eta, N);
+  add(c.ring, de, 3 * N);
+  const int rc = staged(
+      ctx, n_out, 1, [](size_t, size_t, double *) {},
+      [&](size_t first, size_t count, double *buf) {
+        hipLaunchKernelGGL((k_state_out<T>), dim3(unsigned((count + kBlock - 1) / kBlock)), dim3(kBlock), 0,
+                           ctx->stream, f, c, (long long)first, int(count), buf);
+      },
+      [&](size_t first, size_t count, const double *buf) {
+        for (int q = 0; q < n_seg; q++) {
+          const size_t lo = std::max(first, seg[q].lo), hi = std::min(first + count, seg[q].lo + seg[q].n);
+          if (lo < hi) std::memcpy(seg[q].dst + (lo - seg[q].lo), buf + (lo - first), (hi - lo) * sizeof(double));
+        }
+      });
+  if (rc) return rc;
+  // entries of a history as it was set (none set: zeros)
+  auto as_set = [&](double *ds, size_t n, const std::vector<double> &keep) {
+    if (!ds) return;
+    if (k == 0) {
+      if (keep.empty()) std::fill(ds, ds + 3 * n, 0.0);
+      else std::copy(keep.begin(), keep.end(), ds);
+    } else if (euler && !keep.empty()) {
+      for (size_t i = 0; i < n; i++) ds[3 * i + 1] = keep[3 * i + 1];
+    }
+  };
+  as_set(dv, E, ctx->init_hist_v[b]);
+  as_set(de, N, ctx->init_hist_e[b]);
   return ODIS_OK;
 }
 
@@ -2924,7 +3114,6 @@ static int get_state_impl(odis_ctx *ctx, int inst, double *v, double *dvdt, doub
   if (inst < 0 || inst >= ctx->B) return fail(ctx, ODIS_E_RANGE, "instance out of range");
   const int rc = il_out_any(ctx);
   if (rc) return rc;
-  CK(hipStreamSynchronize(ctx->stream));
   if (iter) *iter = ctx->step;
   return ctx->precision == ODIS_FP64 ? get_state_t(ctx, ctx->d, inst, v, dvdt, eta, detadt, ctx->step)
                                      : get_state_t(ctx, ctx->f, inst, v, dvdt, eta, detadt, ctx->step);
@@ -3867,40 +4056,33 @@ static int res_setup(odis_ctx *ctx) {
                o_face = put(h.face), o_fcell = put(h.fcell), o_bface = put(h.bface), o_bcell = put(h.bcell),
                o_bhalo = put(h.bhalo), o_bpeer = put(h.bpeer), o_cyc = all.size();
   const size_t bytes = all.size() * sizeof(int) + h.cyc.size() * sizeof(unsigned short);
-  auto alloc = [&](void **dst, size_t n) -> int {
-    if (hipMalloc(dst, n) != hipSuccess) return fail(ctx, ODIS_E_NOMEM, "hipMalloc of the resident step");
-    r.allocs.push_back(*dst);
-    return ODIS_OK;
-  };
   r.chunk = int(std::max<size_t>(size_t(kResMinSteps),
                                  std::min<size_t>(size_t(std::min(ctx->chunk, 1024)),
                                                   kResPartBytes / (sizeof(double) * size_t(B) * W))));
   r.chunk = std::min(r.chunk, ctx->chunk);
-  void *ops = nullptr, *work = nullptr, *part = nullptr;
+  // one buffer: control words, inboxes, dissipation partials, patch arrays
   const size_t mail = size_t(r.ipl) * kResDepth * S * kResPlanes<T> * sizeof(uint4v);
-  int rc;
-  if ((rc = alloc(&ops, bytes)) || (rc = alloc(&work, 64 + mail)) ||
-      (rc = alloc(&part, size_t(B) * r.chunk * W * sizeof(double))))
-    return rc;
-  CK(hipMemcpy(ops, all.data(), all.size() * sizeof(int), hipMemcpyHostToDevice));
-  CK(hipMemcpy(static_cast<int *>(ops) + o_cyc, h.cyc.data(), h.cyc.size() * sizeof(unsigned short),
-               hipMemcpyHostToDevice));
+  const size_t part = size_t(B) * r.chunk * W * sizeof(double);
+  void *buf = nullptr;
+  if (hipMalloc(&buf, 64 + mail + part + bytes) != hipSuccess)
+    return fail(ctx, ODIS_E_NOMEM, "hipMalloc of the resident step");
+  r.allocs.push_back(buf);
+  char *const work = static_cast<char *>(buf), *const ops = work + 64 + mail + part;
   CK(hipMemset(work, 0, 64 + mail));
-  if (!r.status) {
-    void *st = nullptr;
-    CK(hipHostMalloc(&st, 64, hipHostMallocDefault));
-    r.status = static_cast<unsigned *>(st);
-  }
+  CK(hipMemcpy(ops, all.data(), all.size() * sizeof(int), hipMemcpyHostToDevice));
+  CK(hipMemcpy(ops + o_cyc * sizeof(int), h.cyc.data(), h.cyc.size() * sizeof(unsigned short),
+               hipMemcpyHostToDevice));
+  r.status = reinterpret_cast<unsigned *>(ctx->coef_host[0] + ctx->coef_doubles);
   *r.status = 0;
   CK(hipDeviceSynchronize());
-  const int *base = static_cast<const int *>(ops);
+  const int *base = reinterpret_cast<const int *>(ops);
   r.cptr = base + o_cptr, r.fptr = base + o_fptr, r.bptr = base + o_bptr, r.cell = base + o_cell;
   r.face = base + o_face, r.fcell = base + o_fcell, r.bface = base + o_bface, r.bcell = base + o_bcell;
   r.bhalo = base + o_bhalo, r.bpeer = base + o_bpeer;
   r.cyc = reinterpret_cast<const unsigned short *>(base + o_cyc);
-  r.ctl = static_cast<unsigned long long *>(work);
-  r.mail = reinterpret_cast<uint4v *>(static_cast<char *>(work) + 64);
-  r.part = static_cast<double *>(part);
+  r.ctl = reinterpret_cast<unsigned long long *>(work);
+  r.mail = reinterpret_cast<uint4v *>(work + 64);
+  r.part = reinterpret_cast<double *>(work + 64 + mail);
   r.W = W;
   r.variant = v;
   r.slots = S;
@@ -4188,10 +4370,10 @@ static int get_dissipation_series_impl(odis_ctx *ctx, int inst, long long first,
   // series[k] exists for max(series_lo, step - cap) <= k < step
   if (first < ctx->series_lo || first + count > ctx->step || first < ctx->step - ctx->cap)
     return fail(ctx, ODIS_E_RANGE, "series range not available");
-  std::vector<double> all(ctx->cap);
-  CK(hipMemcpy(all.data(), ctx->series + size_t(inst) * ctx->cap, sizeof(double) * ctx->cap,
-               hipMemcpyDeviceToHost));
-  for (int k = 0; k < count; k++) out[k] = all[size_t((first + k) % ctx->cap)];
+  const double *ring = ctx->series + size_t(inst) * ctx->cap;
+  const int at = int(first % ctx->cap), head = std::min(count, ctx->cap - at);
+  if (head) CK(hipMemcpy(out, ring + at, sizeof(double) * head, hipMemcpyDeviceToHost));
+  if (count > head) CK(hipMemcpy(out + head, ring, sizeof(double) * (count - head), hipMemcpyDeviceToHost));
   return ODIS_OK;
 }
 
@@ -4377,44 +4559,25 @@ extern "C" int odis_retire(odis_ctx *ctx, const int *keep, int n_keep) {
 
 template <typename T>
 static int vel_t(odis_ctx *ctx, Ops<T> &o, int b, const double *normal, double *uv) {
-  const int E = ctx->E;
+  const size_t E = ctx->E;
   const int rc = il_out_any(ctx);
   if (rc) return rc;
-  std::vector<double> nd(size_t(2) * E);
-  for (int r = 0; r < E; r++) {
-    nd[2 * r] = normal[2 * ctx->face_inv[r]];
-    nd[2 * r + 1] = normal[2 * ctx->face_inv[r] + 1];
-  }
-  double *dn = nullptr, *duv = nullptr;
-  CK(hipMalloc(&dn, sizeof(double) * 2 * E));
-  hipError_t e = hipMalloc(&duv, sizeof(double) * 2 * E);
-  if (e != hipSuccess) {
-    (void)hipFree(dn);
-    return fail(ctx, ODIS_E_NOMEM, "hipMalloc");
-  }
-  std::vector<double> h(size_t(2) * E);
-  e = hipMemcpy(dn, nd.data(), sizeof(double) * 2 * E, hipMemcpyHostToDevice);
-  if (e == hipSuccess) {
-    hipLaunchKernelGGL((k_velocity_en<T>), dim3((E + kBlock - 1) / kBlock), dim3(kBlock), 0, ctx->stream, E,
-                       o.tri_idx, o.tri_coef, o.v[ctx->cur] + size_t(b) * E, dn, duv);
-    e = hipGetLastError();
-  }
-  if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-  if (e == hipSuccess) e = hipMemcpy(h.data(), duv, sizeof(double) * 2 * E, hipMemcpyDeviceToHost);
-  (void)hipFree(dn);
-  (void)hipFree(duv);
-  if (e != hipSuccess) return fail(ctx, ODIS_E_HIP, hipGetErrorString(e));
-  for (int r = 0; r < E; r++) {
-    uv[2 * ctx->face_inv[r]] = h[2 * r];
-    uv[2 * ctx->face_inv[r] + 1] = h[2 * r + 1];
-  }
-  return ODIS_OK;
+  return staged(
+      ctx, E, 4, [&](size_t first, size_t count, double *buf) { std::memcpy(buf, normal + 2 * first, 16 * count); },
+      [&](size_t first, size_t count, double *buf) {
+        hipLaunchKernelGGL((k_velocity_en<T>), dim3(unsigned((count + kBlock - 1) / kBlock)), dim3(kBlock), 0,
+                           ctx->stream, int(E), int(first), int(count), ctx->face_perm_dev, o.tri_idx, o.tri_coef,
+                           o.v[ctx->cur] + b * E, reinterpret_cast<const double2 *>(buf),
+                           reinterpret_cast<double2 *>(buf + 2 * count));
+      },
+      [&](size_t first, size_t count, const double *buf) {
+        std::memcpy(uv + 2 * first, buf + 2 * count, 16 * count);
+      });
 }
 
 static int get_velocity_en_impl(odis_ctx *ctx, int inst, const double *face_normal, double *uv) {
   if (!ctx || !face_normal || !uv) return ODIS_E_INVALID;
   if (inst < 0 || inst >= ctx->B) return fail(ctx, ODIS_E_RANGE, "instance out of range");
-  CK(hipStreamSynchronize(ctx->stream));
   return ctx->precision == ODIS_FP64 ? vel_t(ctx, ctx->d, inst, face_normal, uv)
                                      : vel_t(ctx, ctx->f, inst, face_normal, uv);
 }
@@ -4670,7 +4833,7 @@ static int rbf_set_impl(odis_ctx *ctx, int n_rows, int n_cols, const int *row_pt
   for (void *p : ctx->rbf_allocs) (void)hipFree(p);
   ctx->rbf_allocs.clear();
   ctx->rbf_idx = nullptr;
-  ctx->rbf_w = ctx->rbf_out = nullptr;
+  ctx->rbf_w = nullptr;
   auto up = [&](void **dst, const void *src, size_t bytes) -> int {
     void *p = nullptr;
     CK(hipMalloc(&p, bytes));
@@ -4681,13 +4844,11 @@ static int rbf_set_impl(odis_ctx *ctx, int n_rows, int n_cols, const int *row_pt
   };
   // the operator is in use (rbf_idx set) only once all of it is in place
   int *d_idx = nullptr;
-  double *d_w = nullptr, *d_out = nullptr;
+  double *d_w = nullptr;
   int rc;
   if ((rc = up(reinterpret_cast<void **>(&d_idx), idx.data(), idx.size() * sizeof(int)))) return rc;
   if ((rc = up(reinterpret_cast<void **>(&d_w), w.data(), w.size() * sizeof(double)))) return rc;
-  if ((rc = up(reinterpret_cast<void **>(&d_out), nullptr, size_t(3) * N * sizeof(double)))) return rc;
   ctx->rbf_w = d_w;
-  ctx->rbf_out = d_out;
   ctx->rbf_idx = d_idx;
   return ODIS_OK;
 }
@@ -4703,23 +4864,21 @@ static int velocity_xyz_impl(odis_ctx *ctx, int inst, double *xyz) {
   if (!ctx->rbf_idx) return fail(ctx, ODIS_E_INVALID, "no RBF operator set");
   const int rc = il_out_any(ctx);
   if (rc) return rc;
-  const int N = ctx->N;
-  const dim3 grid((N + kBlock - 1) / kBlock), blk(kBlock);
-  if (ctx->precision == ODIS_FP64)
-    hipLaunchKernelGGL((k_velocity_xyz<double>), grid, blk, 0, ctx->stream, N, ctx->rbf_idx, ctx->rbf_w,
-                       ctx->d.v[ctx->cur] + size_t(inst) * ctx->E, ctx->rbf_out);
-  else
-    hipLaunchKernelGGL((k_velocity_xyz<float>), grid, blk, 0, ctx->stream, N, ctx->rbf_idx, ctx->rbf_w,
-                       ctx->f.v[ctx->cur] + size_t(inst) * ctx->E, ctx->rbf_out);
-  CK(hipGetLastError());
-  std::vector<double> h(size_t(3) * N);
-  CK(hipMemcpyAsync(h.data(), ctx->rbf_out, sizeof(double) * 3 * N, hipMemcpyDeviceToHost, ctx->stream));
-  CK(hipStreamSynchronize(ctx->stream));
-  for (int r = 0; r < N; r++) {
-    const int i = ctx->cell_inv[r];
-    for (int c = 0; c < 3; c++) xyz[3 * i + c] = h[size_t(c) * N + r];
-  }
-  return ODIS_OK;
+  const size_t N = ctx->N;
+  return staged(
+      ctx, 3 * N, 1, [](size_t, size_t, double *) {},
+      [&](size_t first, size_t count, double *buf) {
+        const dim3 grid(unsigned((count + kBlock - 1) / kBlock)), blk(kBlock);
+        if (ctx->precision == ODIS_FP64)
+          hipLaunchKernelGGL((k_velocity_xyz<double>), grid, blk, 0, ctx->stream, int(N), int(first), int(count),
+                             ctx->cell_perm_dev, ctx->rbf_idx, ctx->rbf_w, ctx->d.v[ctx->cur] + size_t(inst) * ctx->E,
+                             buf);
+        else
+          hipLaunchKernelGGL((k_velocity_xyz<float>), grid, blk, 0, ctx->stream, int(N), int(first), int(count),
+                             ctx->cell_perm_dev, ctx->rbf_idx, ctx->rbf_w, ctx->f.v[ctx->cur] + size_t(inst) * ctx->E,
+                             buf);
+      },
+      [&](size_t first, size_t count, const double *buf) { std::memcpy(xyz + first, buf, count * sizeof(double)); });
 }
 
 extern "C" int odis_velocity_xyz(odis_ctx *ctx, int inst, double *xyz) {
