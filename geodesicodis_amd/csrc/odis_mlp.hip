@@ -4,12 +4,24 @@
 // rest, a file or its analytic solution (src/initialConditions.cpp:19-206).
 //
 // All products (forward X W^T, weight gradients dZ^T X, input gradients
-// dZ W) run on one FP32 matrix-core kernel, k_mlp_gemm: a 64 x 64 tile per
-// workgroup, 4 waves of 32 x 32, v_mfma_f32_16x16x4f32 over K in LDS stages
-// of 16, with the bias and tanh fused into the forward epilogue.  Loss
-// (mean squared error / 2), bias gradients, Adam and the minibatch gather
-// are small elementwise kernels.  Sums that give the loss and the bias
-// gradients run in a fixed order, so a training run is deterministic.
+// dZ W) run on one FP32 matrix-core tile, gemm_tile: 32 x 32 per workgroup,
+// 4 waves of 16 x 16, v_mfma_f32_16x16x4f32 over K in double-buffered LDS
+// stages of 128, the next stage's loads under way during a stage.  Why so
+// small a tile: a minibatch of 256 rows and 256 columns is only 64 of them,
+// and the longest product (input gradient of the output layer, K = 1732) is
+// one chain of 433 dependent products per wave whatever the tile.  The order
+// of the sums over K is ascending, one accumulator per element.
+//
+// A minibatch is launches and latency more than arithmetic (1 GFLOP, 7 us at
+// the card's FP32 rate), so its kernels are few: bias and tanh are in the
+// forward epilogue; one launch per layer goes backward (input gradient with
+// the tanh derivative of the layer below, weight gradient, bias gradient as
+// ranges of workgroups); the loss reads its targets through the minibatch's
+// indices.  With 64 x 64 tiles staged 16 entries deep, a thread per column of
+// the bias gradients and 29 launches, a minibatch of 256 rows of the 2 -> 4 x
+// 256 -> 1732 network took 960 us; now 135 in 13 launches.
+// Sums that give the loss and the bias gradients run in a fixed order, so a
+// training run is deterministic.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -39,70 +51,151 @@ int mlp_fail(int code, const std::string &msg) {
     if (e_ != hipSuccess) return mlp_fail(ODIS_E_HIP, std::string(#x) + ": " + hipGetErrorString(e_)); \
   } while (0)
 
-constexpr int kTile = 64, kKs = 16, kThreads = 256;
+constexpr int kTile = 32, kKs = 128, kThreads = 256;
+constexpr int kPitch = kKs + 4;  // LDS row pitch: a fragment's 16 rows x 4 entries fall on 64 banks
+constexpr int kPer = kTile * kKs / kThreads;  // entries of an operand stage per thread
+constexpr int kPartBlocks = kThreads;         // workgroups of the loss: one partial per thread of add_loss
 
-// C[m][n] = sum_k A(m, k) B(k, n) (+ bias[n], then tanh when ACT).
-// A(m, k) = TA ? A[k * lda + m] : A[m * lda + k]; B(k, n) = TB ? B[n * ldb + k]
-// : B[k * ldb + n].  Out-of-range operands read as 0, out-of-range results
-// are not stored.  Wave w of the workgroup computes rows 32 (w / 2) and
-// columns 32 (w % 2) of the tile as 2 x 2 blocks of 16 x 16; lane l of a
-// block holds A(l % 16, l / 16), B(l / 16, l % 16) per product and
-// C(4 (l / 16) + r, l % 16), r = 0..3, of the result.
-template <bool TA, bool TB, int EPI>  // EPI 0: store, 1: + bias, 2: + bias, tanh
-__global__ __launch_bounds__(kThreads) void k_mlp_gemm(int M, int N, int K, const float *__restrict__ A, int lda,
-                                                       const float *__restrict__ B, int ldb,
-                                                       const float *__restrict__ bias, float *__restrict__ C,
-                                                       int ldc) {
-  __shared__ float As[kTile][kKs + 1];
-  __shared__ float Bs[kKs][kTile + 1];
-  const int m0 = blockIdx.y * kTile, n0 = blockIdx.x * kTile;
+// LDS of a tile: two stages of both operands, [stage][operand][row][k]
+struct GemmLds {
+  float s[2][2][kTile][kPitch];
+};
+
+// Entry (r, k) of an operand is X[(r0 + r) * ld + k0 + k] (KC: k contiguous)
+// or X[(k0 + k) * ld + r0 + r]; out of range 0.  Threads run along memory.
+template <bool KC>
+__device__ __forceinline__ void load_stage(const float *__restrict__ X, int ld, int r0, int R, int k0, int K,
+                                           float (&x)[kPer]) {
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    const int q = threadIdx.x + j * kThreads;
+    const int r = r0 + (KC ? q / kKs : q % kTile), k = k0 + (KC ? q % kKs : q / kTile);
+    x[j] = (r < R && k < K) ? X[KC ? (size_t)r * ld + k : (size_t)k * ld + r] : 0.f;
+  }
+}
+template <bool KC>
+__device__ __forceinline__ void store_stage(float (*s)[kPitch], const float (&x)[kPer]) {
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    const int q = threadIdx.x + j * kThreads;
+    s[KC ? q / kKs : q % kTile][KC ? q % kKs : q / kTile] = x[j];
+  }
+}
+
+// Tile (bx, by) of C[m][n] = sum_k A(m, k) B(k, n).  A(m, k) = TA ?
+// A[k * lda + m] : A[m * lda + k]; B(k, n) = TB ? B[n * ldb + k] : B[k * ldb + n].
+// EPI 0: store, 1: + aux[n] (bias), 2: tanh of that, 3: times 1 - aux[m][n]^2
+// (the tanh derivative through the layer's output, [M][ldc]).  Out-of-range
+// operands read as 0, out-of-range results are not stored.  Lane l of a wave
+// holds A(l % 16, l / 16), B(l / 16, l % 16) per product and C(4 (l / 16) + r,
+// l % 16), r = 0..3, of the result.
+template <bool TA, bool TB, int EPI>
+__device__ __forceinline__ void gemm_tile(GemmLds &lds, int bx, int by, int M, int N, int K,
+                                          const float *__restrict__ A, int lda, const float *__restrict__ B, int ldb,
+                                          const float *__restrict__ aux, float *__restrict__ C, int ldc) {
+  const int m0 = by * kTile, n0 = bx * kTile;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
+  const int wm = (wave >> 1) * 16, wn = (wave & 1) * 16, r16 = lane & 15, g = lane >> 4;
   typedef float f4 __attribute__((ext_vector_type(4)));
-  f4 acc[2][2];
-  for (int i = 0; i < 2; ++i)
-    for (int j = 0; j < 2; ++j) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
-  for (int k0 = 0; k0 < K; k0 += kKs) {
-    // 1024 elements of each operand tile, 4 per thread
-    for (int q = threadIdx.x; q < kTile * kKs; q += kThreads) {
-      const int r = TA ? q % kTile : q / kKs, c = TA ? q / kTile : q % kKs;  // coalesced along memory
-      const int gm = m0 + r, gk = k0 + c;
-      As[r][c] = (gm < M && gk < K) ? (TA ? A[(size_t)gk * lda + gm] : A[(size_t)gm * lda + gk]) : 0.f;
-      const int rb = TB ? q % kKs : q / kTile, cb = TB ? q / kKs : q % kTile;
-      const int bk = k0 + rb, bn = n0 + cb;
-      Bs[rb][cb] = (bk < K && bn < N) ? (TB ? B[(size_t)bn * ldb + bk] : B[(size_t)bk * ldb + bn]) : 0.f;
+  f4 acc = f4{0.f, 0.f, 0.f, 0.f};
+  float xa[kPer], xb[kPer];
+  load_stage<!TA>(A, lda, m0, M, 0, K, xa);
+  load_stage<TB>(B, ldb, n0, N, 0, K, xb);
+  store_stage<!TA>(lds.s[0][0], xa);
+  store_stage<TB>(lds.s[0][1], xb);
+  __syncthreads();
+  for (int k0 = 0, st = 0; k0 < K; k0 += kKs, st ^= 1) {
+    const bool more = k0 + kKs < K;
+    if (more) {
+      load_stage<!TA>(A, lda, m0, M, k0 + kKs, K, xa);
+      load_stage<TB>(B, ldb, n0, N, k0 + kKs, K, xb);
     }
-    __syncthreads();
+    const float *pa = &lds.s[st][0][wm + r16][g], *pb = &lds.s[st][1][wn + r16][g];
+    const int steps = min(kKs, K - k0);
+    if (steps == kKs) {
 #pragma unroll
-    for (int kk = 0; kk < kKs; kk += 4) {
-      float a[2], b[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) a[i] = As[wm + 16 * i + (lane & 15)][kk + (lane >> 4)];
-#pragma unroll
-      for (int j = 0; j < 2; ++j) b[j] = Bs[kk + (lane >> 4)][wn + 16 * j + (lane & 15)];
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[j], acc[i][j], 0, 0, 0);
+      for (int kk = 0; kk < kKs; kk += 4) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(pa[kk], pb[kk], acc, 0, 0, 0);
+    } else {
+      for (int kk = 0; kk < steps; kk += 4) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(pa[kk], pb[kk], acc, 0, 0, 0);
+    }
+    if (more) {
+      store_stage<!TA>(lds.s[st ^ 1][0], xa);
+      store_stage<TB>(lds.s[st ^ 1][1], xb);
     }
     __syncthreads();
   }
+  const int col = n0 + wn + r16;
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int col = n0 + wn + 16 * j + (lane & 15);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = m0 + wm + 16 * i + 4 * (lane >> 4) + r;
-        if (row < M && col < N) {
-          float x = acc[i][j][r];
-          if (EPI >= 1) x += bias[col];
-          if (EPI == 2) x = tanhf(x);
-          C[(size_t)row * ldc + col] = x;
-        }
+  for (int r = 0; r < 4; ++r) {
+    const int row = m0 + wm + 4 * g + r;
+    if (row < M && col < N) {
+      float x = acc[r];
+      if (EPI == 1 || EPI == 2) x += aux[col];
+      if (EPI == 2) x = tanhf(x);
+      if (EPI == 3) {
+        const float a = aux[(size_t)row * ldc + col];
+        x *= 1.f - a * a;
       }
+      C[(size_t)row * ldc + col] = x;
     }
+  }
+}
+
+// forward: C = act(A W^T + bias)
+template <int EPI>
+__global__ __launch_bounds__(kThreads) void k_mlp_forward(int M, int N, int K, const float *__restrict__ A,
+                                                          const float *__restrict__ W,
+                                                          const float *__restrict__ bias, float *__restrict__ C) {
+  __shared__ GemmLds lds;
+  const int cols = (N + kTile - 1) / kTile, t = blockIdx.x;
+  gemm_tile<false, true, EPI>(lds, t % cols, t / cols, M, N, K, A, K, W, K, bias, C, N);
+}
+
+// Bias gradient db[j] = sum over the rows of dZ[., j], in row order: 16
+// columns per workgroup, 256 rows at a time through LDS.
+__device__ __forceinline__ void colsum_tile(GemmLds &lds, int bx, int M, int N, const float *__restrict__ dZ,
+                                            float *__restrict__ db) {
+  constexpr int C = 16, R = kThreads;
+  float(*s)[C + 1] = reinterpret_cast<float(*)[C + 1]>(&lds);
+  static_assert(sizeof(float) * R * (C + 1) <= sizeof(GemmLds), "column sums fit the tile's LDS");
+  const int c = threadIdx.x % C, r = threadIdx.x / C, col = bx * C + c;
+  float sum = 0.f;
+  for (int m0 = 0; m0 < M; m0 += R) {
+#pragma unroll
+    for (int j = 0; j < C; ++j) {
+      const int m = m0 + r + j * (kThreads / C);
+      s[r + j * (kThreads / C)][c] = (m < M && col < N) ? dZ[(size_t)m * N + col] : 0.f;
+    }
+    __syncthreads();
+    if (r == 0) {
+      const int rows = min(R, M - m0);
+#pragma unroll 16
+      for (int m = 0; m < rows; ++m) sum += s[m][c];
+    }
+    __syncthreads();
+  }
+  if (r == 0 && col < N) db[col] = sum;
+}
+
+// One layer backward, from dZ [n][no] (gradient of its pre-activation
+// output): workgroups [0, n_dx) the tiles of dIn = (dZ W) (1 - in^2) [n][ni]
+// (the layer below's dZ; none for the first layer), the next n_dw those of
+// dW = dZ^T in [no][ni], the rest 16 columns of db each.
+__global__ __launch_bounds__(kThreads) void k_mlp_backward(int n, int no, int ni, int n_dx, int n_dw,
+                                                           const float *__restrict__ dZ,
+                                                           const float *__restrict__ W,
+                                                           const float *__restrict__ in, float *__restrict__ dIn,
+                                                           float *__restrict__ dW, float *__restrict__ db) {
+  __shared__ GemmLds lds;
+  int t = blockIdx.x;
+  const int cols = (ni + kTile - 1) / kTile;
+  if (t < n_dx) {
+    gemm_tile<false, false, 3>(lds, t % cols, t / cols, n, ni, no, dZ, no, W, ni, in, dIn, ni);
+  } else if ((t -= n_dx) < n_dw) {
+    gemm_tile<true, false, 0>(lds, t % cols, t / cols, no, ni, n, dZ, no, in, ni, nullptr, dW, ni);
+  } else {
+    colsum_tile(lds, t - n_dw, n, no, dZ, db);
+  }
 }
 
 // rows idx[m] of the data set into a contiguous minibatch
@@ -113,14 +206,17 @@ __global__ __launch_bounds__(kThreads) void k_mlp_gather(int n, int w, const int
 }
 
 // dY = (Y - T) / count and a fixed-order partial of the squared error per
-// workgroup: loss = sum (Y - T)^2 / (2 count)
-__global__ __launch_bounds__(kThreads) void k_mlp_mse(size_t total, double count, const float *__restrict__ Y,
-                                                       const float *__restrict__ T, float *__restrict__ dY,
-                                                       double *__restrict__ part) {
+// workgroup: loss = sum (Y - T)^2 / (2 count); row m of T is row idx[m] of
+// the data set's targets
+__global__ __launch_bounds__(kThreads) void k_mlp_mse(int n, int w, double count, const float *__restrict__ Y,
+                                                       const int *__restrict__ idx, const float *__restrict__ T,
+                                                       float *__restrict__ dY, double *__restrict__ part) {
   __shared__ double sh[kThreads];
   double s = 0.0;
+  const size_t total = size_t(n) * w;
   for (size_t i = (size_t)blockIdx.x * kThreads + threadIdx.x; i < total; i += (size_t)gridDim.x * kThreads) {
-    const double d = double(Y[i]) - double(T[i]);
+    const size_t row = (i >> 32) ? i / w : unsigned(i) / unsigned(w), col = i - row * w;
+    const double d = double(Y[i]) - double(T[(size_t)idx[row] * w + col]);
     s += d * d;
     dY[i] = float(d / count);
   }
@@ -133,36 +229,29 @@ __global__ __launch_bounds__(kThreads) void k_mlp_mse(size_t total, double count
   if (threadIdx.x == 0) part[blockIdx.x] = sh[0] / (2.0 * count);
 }
 
-// acc[0] += sum of the partials (one thread, fixed order)
-__global__ void k_mlp_sum(int n, const double *__restrict__ part, double *__restrict__ acc) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
+// acc[0] += sum of the loss partials, in order
+__device__ __forceinline__ void add_loss(const double *__restrict__ part, double *__restrict__ acc) {
+  __shared__ double sh[kPartBlocks];
+  sh[threadIdx.x] = part[threadIdx.x];
+  __syncthreads();
+  if (threadIdx.x == 0) {
     double s = 0.0;
-    for (int i = 0; i < n; ++i) s += part[i];
+#pragma unroll 16
+    for (int i = 0; i < kPartBlocks; ++i) s += sh[i];
     acc[0] += s;
   }
 }
-
-// dZ = dA (1 - A^2), the tanh derivative through its output
-__global__ __launch_bounds__(kThreads) void k_mlp_dtanh(size_t total, const float *__restrict__ A,
-                                                         float *__restrict__ dZ) {
-  const size_t i = (size_t)blockIdx.x * kThreads + threadIdx.x;
-  if (i < total) dZ[i] *= 1.f - A[i] * A[i];
+__global__ __launch_bounds__(kThreads) void k_mlp_sum(const double *__restrict__ part, double *__restrict__ acc) {
+  add_loss(part, acc);
 }
 
-// db[j] = sum over rows of dZ[., j] (fixed order per column)
-__global__ __launch_bounds__(kThreads) void k_mlp_colsum(int M, int N, const float *__restrict__ dZ,
-                                                          float *__restrict__ db) {
-  const int j = blockIdx.x * kThreads + threadIdx.x;
-  if (j >= N) return;
-  float s = 0.f;
-  for (int m = 0; m < M; ++m) s += dZ[(size_t)m * N + j];
-  db[j] = s;
-}
-
-// Adam (Kingma & Ba) with bias-corrected moments
+// Adam (Kingma & Ba) with bias-corrected moments; the first workgroup also
+// adds the minibatch's loss
 __global__ __launch_bounds__(kThreads) void k_mlp_adam(int n, float lr, float b1, float b2, float eps, float c1,
                                                         float c2, const float *__restrict__ g, float *__restrict__ p,
-                                                        float *__restrict__ m, float *__restrict__ v) {
+                                                        float *__restrict__ m, float *__restrict__ v,
+                                                        const double *__restrict__ part, double *__restrict__ acc) {
+  if (blockIdx.x == 0) add_loss(part, acc);
   const int i = blockIdx.x * kThreads + threadIdx.x;
   if (i >= n) return;
   const float gi = g[i];
@@ -183,7 +272,6 @@ struct odis_mlp {
   int cap = 0;                        // rows the activation buffers hold
   std::vector<float *> act;           // act[0] = input batch, act[l + 1] = output of layer l
   float *dA = nullptr, *dB = nullptr; // gradient buffers [cap][max width]
-  float *tgt = nullptr;               // target batch [cap][n_out]
   double *part = nullptr, *acc = nullptr;
   int n_data = 0;
   float *X = nullptr, *Y = nullptr;   // data set on the device
@@ -195,7 +283,6 @@ struct odis_mlp {
 
 namespace {
 
-constexpr int kPartBlocks = 64;
 
 template <typename T>
 int mlp_alloc(odis_mlp *m, T **p, size_t count) {
@@ -224,7 +311,7 @@ int ensure_capacity(odis_mlp *m, int rows) {
       if (it != m->allocs.end()) m->allocs.erase(it);
       (void)hipFree(a);
     }
-  for (float **b : {&m->dA, &m->dB, &m->tgt})
+  for (float **b : {&m->dA, &m->dB})
     if (*b) {
       auto it = std::find(m->allocs.begin(), m->allocs.end(), static_cast<void *>(*b));
       if (it != m->allocs.end()) m->allocs.erase(it);
@@ -237,55 +324,37 @@ int ensure_capacity(odis_mlp *m, int rows) {
   for (int l = 0; l <= m->depth && !rc; ++l) rc = mlp_alloc(m, &m->act[l + 1], size_t(rows) * m->dout[l]);
   if (!rc) rc = mlp_alloc(m, &m->dA, size_t(rows) * wmax);
   if (!rc) rc = mlp_alloc(m, &m->dB, size_t(rows) * wmax);
-  if (!rc) rc = mlp_alloc(m, &m->tgt, size_t(rows) * m->n_out);
   if (rc) return rc;
   m->cap = rows;
   return ODIS_OK;
-}
-
-template <bool TA, bool TB, int EPI>
-void gemm(odis_mlp *m, int M, int N, int K, const float *A, int lda, const float *B, int ldb, const float *bias,
-          float *C, int ldc) {
-  const dim3 grid((N + kTile - 1) / kTile, (M + kTile - 1) / kTile);
-  hipLaunchKernelGGL((k_mlp_gemm<TA, TB, EPI>), grid, dim3(kThreads), 0, m->stream, M, N, K, A, lda, B, ldb, bias,
-                     C, ldc);
 }
 
 // forward pass of the n rows in act[0]; act[l + 1] = layer l's output
 void forward(odis_mlp *m, int n) {
   for (int l = 0; l <= m->depth; ++l) {
     const float *W = m->p + m->woff[l], *b = m->p + m->boff[l];
+    const int no = m->dout[l], ni = m->din[l];
+    const dim3 grid(unsigned((no + kTile - 1) / kTile) * unsigned((n + kTile - 1) / kTile));
     if (l < m->depth)
-      gemm<false, true, 2>(m, n, m->dout[l], m->din[l], m->act[l], m->din[l], W, m->din[l], b, m->act[l + 1],
-                           m->dout[l]);
+      hipLaunchKernelGGL((k_mlp_forward<2>), grid, dim3(kThreads), 0, m->stream, n, no, ni, m->act[l], W, b,
+                         m->act[l + 1]);
     else
-      gemm<false, true, 1>(m, n, m->dout[l], m->din[l], m->act[l], m->din[l], W, m->din[l], b, m->act[l + 1],
-                           m->dout[l]);
+      hipLaunchKernelGGL((k_mlp_forward<1>), grid, dim3(kThreads), 0, m->stream, n, no, ni, m->act[l], W, b,
+                         m->act[l + 1]);
   }
 }
 
-// loss of act[depth + 1] against tgt added to acc[0], gradients into g
-void backward(odis_mlp *m, int n) {
-  const size_t tot = size_t(n) * m->n_out;
-  hipLaunchKernelGGL(k_mlp_mse, dim3(kPartBlocks), dim3(kThreads), 0, m->stream, tot, double(tot),
-                     m->act[m->depth + 1], m->tgt, m->dA, m->part);
-  hipLaunchKernelGGL(k_mlp_sum, dim3(1), dim3(64), 0, m->stream, kPartBlocks, m->part, m->acc);
+// loss partials of act[depth + 1] against the rows idx of the targets, gradients into g
+void backward(odis_mlp *m, int n, const int *idx) {
+  hipLaunchKernelGGL(k_mlp_mse, dim3(kPartBlocks), dim3(kThreads), 0, m->stream, n, m->n_out,
+                     double(size_t(n) * m->n_out), m->act[m->depth + 1], idx, m->Y, m->dA, m->part);
   float *dcur = m->dA, *dnext = m->dB;  // dcur: gradient of layer l's pre-activation output
   for (int l = m->depth; l >= 0; --l) {
-    const int no = m->dout[l], ni = m->din[l];
-    if (l < m->depth) {
-      const size_t t2 = size_t(n) * no;
-      hipLaunchKernelGGL(k_mlp_dtanh, dim3(unsigned((t2 + kThreads - 1) / kThreads)), dim3(kThreads), 0, m->stream,
-                         t2, m->act[l + 1], dcur);
-    }
-    // dW_l = dZ^T act[l]  ([no][ni]), db_l = column sums of dZ
-    gemm<true, false, 0>(m, no, ni, n, dcur, no, m->act[l], ni, nullptr, m->g + m->woff[l], ni);
-    hipLaunchKernelGGL(k_mlp_colsum, dim3((no + kThreads - 1) / kThreads), dim3(kThreads), 0, m->stream, n, no,
-                       dcur, m->g + m->boff[l]);
-    if (l > 0) {  // d act[l] = dZ W_l  ([n][ni])
-      gemm<false, false, 0>(m, n, ni, no, dcur, no, m->p + m->woff[l], ni, nullptr, dnext, ni);
-      std::swap(dcur, dnext);
-    }
+    const int no = m->dout[l], ni = m->din[l], cols = (ni + kTile - 1) / kTile;
+    const int n_dx = l > 0 ? cols * ((n + kTile - 1) / kTile) : 0, n_dw = cols * ((no + kTile - 1) / kTile);
+    hipLaunchKernelGGL(k_mlp_backward, dim3(n_dx + n_dw + (no + 15) / 16), dim3(kThreads), 0, m->stream, n, no, ni,
+                       n_dx, n_dw, dcur, m->p + m->woff[l], m->act[l], dnext, m->g + m->woff[l], m->g + m->boff[l]);
+    std::swap(dcur, dnext);
   }
 }
 
@@ -434,10 +503,8 @@ namespace {
 int batch_grad(odis_mlp *m, int n, const int *idx_dev) {
   const unsigned gx = unsigned((size_t(n) * m->n_in + kThreads - 1) / kThreads);
   hipLaunchKernelGGL(k_mlp_gather, dim3(gx), dim3(kThreads), 0, m->stream, n, m->n_in, idx_dev, m->X, m->act[0]);
-  const unsigned gy = unsigned((size_t(n) * m->n_out + kThreads - 1) / kThreads);
-  hipLaunchKernelGGL(k_mlp_gather, dim3(gy), dim3(kThreads), 0, m->stream, n, m->n_out, idx_dev, m->Y, m->tgt);
   forward(m, n);
-  backward(m, n);
+  backward(m, n, idx_dev);
   MCK(hipGetLastError());
   return ODIS_OK;
 }
@@ -456,6 +523,8 @@ extern "C" int odis_mlp_loss_grad(odis_mlp *m, int n, const int *idx, double *lo
     MCK(hipMemcpyAsync(m->idx, idx, size_t(n) * sizeof(int), hipMemcpyHostToDevice, m->stream));
     MCK(hipMemsetAsync(m->acc, 0, sizeof(double), m->stream));
     if ((rc = batch_grad(m, n, m->idx))) return rc;
+    hipLaunchKernelGGL(k_mlp_sum, dim3(1), dim3(kThreads), 0, m->stream, m->part, m->acc);
+    MCK(hipGetLastError());
     MCK(hipMemcpyAsync(loss, m->acc, sizeof(double), hipMemcpyDeviceToHost, m->stream));
     if (grad) MCK(hipMemcpyAsync(grad, m->g, m->n_params * sizeof(float), hipMemcpyDeviceToHost, m->stream));
     MCK(hipStreamSynchronize(m->stream));
@@ -494,7 +563,7 @@ extern "C" int odis_mlp_train(odis_mlp *m, int epochs, int batch, float lr_start
         const float c1 = float(1.0 - std::pow(0.9, double(m->adam_t)));
         const float c2 = float(1.0 - std::pow(0.999, double(m->adam_t)));
         hipLaunchKernelGGL(k_mlp_adam, dim3(ga), dim3(kThreads), 0, m->stream, int(m->n_params), lr, b1, b2, 1e-8f,
-                           c1, c2, m->g, m->p, m->m1, m->m2);
+                           c1, c2, m->g, m->p, m->m1, m->m2, m->part, m->acc);
       }
       MCK(hipGetLastError());
       if (epoch_loss) {
