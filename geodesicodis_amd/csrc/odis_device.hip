@@ -1176,10 +1176,9 @@ __global__ __launch_bounds__(kBlock) void k_sh_synth(int K, int N, const double 
 // used for the Gram matrix comes from the same table), cos / sin(m lon) by
 // rotation from cos / sin(lon).  No basis is read from memory: per pass the
 // kernels read 4 values per cell and the coefficient table.
-//   analysis, runtime degree: workgroup (cell chunks, m pair) -- m and
-//     L - m, so every wave has L + 2 degrees -- CPT cells per lane, per
-//     (l, +-m) a wave sum, partials per workgroup added in a fixed order by
-//     k_sh_bsum; degrees 8, 16 and 32 have the pair analysis below;
+//   analysis, runtime degree: workgroup (cell chunks, m), CPT cells per
+//     lane, per (l, +-m) a wave sum, partials per workgroup added in a fixed order by
+//     k_sh_bsum; degrees up to 32 have the pair analysis below;
 //   synthesis: one lane per cell over an m-range.
 
 template <typename T>
@@ -1189,8 +1188,9 @@ __device__ __forceinline__ T wave_sum(T v) {
 }
 
 // Analysis: workgroup = kShWaves waves on kShWaves consecutive cell chunks
-// (64 CPT cells each) and one m pair (m, L - m), so every wave has L + 2
-// degrees.  A wave runs the degrees of each m in blocks of 8: per lane the
+// (64 CPT cells each) and one m.  (A pair m, L - m per workgroup balances the
+// waves, but on small grids the length of a wave's chain is the time: 21
+// workgroups of 10242 cells at degree 12 took 28 us, 39 of one m each 17.6.)  A wave runs the degrees of its m in blocks of 8: per lane the
 // 16 (l, cos / sin) sums over its CPT cells, then a butterfly reduce-scatter
 // over the 64 lanes (xor 1, 2, 4, 8 halving the slots, then xor 16, 32)
 // leaves each of the 16 sums in one lane -- 17 shuffles for 16 sums.  The
@@ -1221,16 +1221,14 @@ __device__ __forceinline__ T reduce_scatter16(T *v, int lane) {
   return r;
 }
 
-template <typename T, int LT, int CPT>
-__global__ __launch_bounds__(64 * kShWaves) void k_sh_analysis_rec(int Lrt, int N, const double *__restrict__ tabm,
+template <typename T, int CPT>
+__global__ __launch_bounds__(64 * kShWaves) void k_sh_analysis_rec(int L, int N, const double *__restrict__ tabm,
                                                                    const double *__restrict__ trig,
                                                                    const T *__restrict__ x, long long x_stride,
                                                                    int n_chunks, double *b_part) {
-  extern __shared__ double red[];  // [kShWaves][2 (L + 2)]
-  const int L = LT > 0 ? LT : Lrt;
+  extern __shared__ double red[];  // [kShWaves][2 (L - m + 1)]
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int n_pairs = L / 2 + 1, n_slot = 2 * (L + 2);
-  const int cblk = blockIdx.x / n_pairs, pair = blockIdx.x % n_pairs;
+  const int cblk = blockIdx.x / (L + 1), m = blockIdx.x % (L + 1), n_slot = 2 * (L - m + 1);
   const int n_cblk = (n_chunks + kShWaves - 1) / kShWaves;
   const int b = blockIdx.y;
   const int chunk = cblk * kShWaves + w;
@@ -1238,37 +1236,53 @@ __global__ __launch_bounds__(64 * kShWaves) void k_sh_analysis_rec(int Lrt, int 
   const double *tsect = tabm, *tf1 = tabm + (L + 1);
   const T *xb = x + b * x_stride;
   double *rw = red + w * n_slot;
-  const int m0 = pair, m1 = L - pair;
   // lane of sum q after reduce_scatter16 is rev4(q); this lane holds q = rev4(lane & 15)
   const int q_lane = ((lane & 1) << 3) | ((lane & 2) << 1) | ((lane & 4) >> 1) | ((lane & 8) >> 3);
   if (chunk < n_chunks) {
-    for (int h = 0; h < 2; ++h) {
-      const int m = h == 0 ? m0 : m1;
-      if (h == 1 && m1 == m0) break;
-      double *slot = rw + (h == 0 ? 0 : 2 * (L - m0 + 1));
+    {
+      double *slot = rw;
       int oab = 2 * (L + 1);
       for (int q = 0; q < m; ++q) oab += 2 * max(0, L - q - 1);
       const double *ab = tabm + oab;  // (a, b) of l = m + 2 + j at 2 j
-      T mu[CPT], xc[CPT], xs[CPT], p1[CPT], p2[CPT];
+      // every cell's operands are under way before the first is used, and a
+      // table entry is loaded once for all of them (one cell after the other,
+      // each waiting for its loads and m table entries: 17.6 us at 10242 cells,
+      // degree 12, instead of 13.9)
+      T mu[CPT], xc[CPT], xs[CPT], p1[CPT], p2[CPT], s[CPT], cl[CPT], sl[CPT];
 #pragma unroll
       for (int j = 0; j < CPT; ++j) {
-        const int i = (chunk * CPT + j) * 64 + lane;
-        const bool ok = i < N;
-        mu[j] = ok ? T(trig[i]) : T(0);
-        const T s = ok ? T(trig[N + i]) : T(0), cl = ok ? T(trig[2 * N + i]) : T(1),
-                sl = ok ? T(trig[3 * N + i]) : T(0);
-        const T xv = ok ? xb[i] : T(0);
-        T cm = T(1), sm = T(0), pmm = T(1);
-        for (int q = 1; q <= m; ++q) {
-          const T c2 = fma(cm, cl, -(sm * sl));
-          sm = fma(sm, cl, cm * sl);
-          cm = c2;
-          pmm = pmm * (T(tsect[q]) * s);
+        const int i = min((chunk * CPT + j) * 64 + lane, N - 1);
+        mu[j] = T(trig[i]);
+        s[j] = T(trig[N + i]);
+        cl[j] = T(trig[2 * N + i]);
+        sl[j] = T(trig[3 * N + i]);
+        p2[j] = xb[i];  // x, until the chain starts
+      }
+#pragma unroll
+      for (int j = 0; j < CPT; ++j) {
+        if ((chunk * CPT + j) * 64 + lane >= N) {
+          mu[j] = s[j] = sl[j] = p2[j] = T(0);
+          cl[j] = T(1);
         }
-        xc[j] = xv * cm;
-        xs[j] = xv * sm;
-        p1[j] = pmm;  // P_{l-1} for l = m + 1 after the first degree
-        p2[j] = T(0);
+        xc[j] = T(1);   // cos, sin (m lon)
+        xs[j] = T(0);
+        p1[j] = T(1);   // P_mm
+      }
+      for (int q = 1; q <= m; ++q) {
+        const T sect = T(tsect[q]);
+#pragma unroll
+        for (int j = 0; j < CPT; ++j) {
+          const T c2 = fma(xc[j], cl[j], -(xs[j] * sl[j]));
+          xs[j] = fma(xs[j], cl[j], xc[j] * sl[j]);
+          xc[j] = c2;
+          p1[j] = p1[j] * (sect * s[j]);
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < CPT; ++j) {
+        xc[j] = p2[j] * xc[j];
+        xs[j] = p2[j] * xs[j];
+        p2[j] = T(0);  // p1: P_{l-1} for l = m + 1 after the first degree
       }
       const int nl = L - m + 1;  // degrees m .. L, index t = l - m
       const T f = T(tf1[m]);
@@ -1319,17 +1333,7 @@ __global__ __launch_bounds__(64 * kShWaves) void k_sh_analysis_rec(int Lrt, int 
   // fixed-order sum over the workgroup's waves, one lane per slot
   const int t = threadIdx.x;
   if (t >= n_slot) return;
-  const int base1 = 2 * (L - m0 + 1);
-  int m, l;
-  if (t < base1) {
-    m = m0;
-    l = m0 + t / 2;
-  } else {
-    if (m1 == m0) return;
-    m = m1;
-    l = m1 + (t - base1) / 2;
-    if (l > L) return;
-  }
+  const int l = m + t / 2;
   const bool sn = (t & 1) != 0;
   if (sn && m == 0) return;
   const int n_w = min(kShWaves, n_chunks - cblk * kShWaves);
@@ -1353,6 +1357,14 @@ __global__ __launch_bounds__(64 * kShWaves) void k_sh_analysis_rec(int Lrt, int 
 // l = m + k at 2 (m (L + 1) - m (m - 1) / 2 + k) (k = 0: beta = 1, S = 1;
 // k = 1: beta = 0), then C_0..C_L.
 // Block sums go to b_part ([B][n_cblk][K]), added by k_sh_bsum.
+//
+// Degrees without a kernel of their own may run in that of the next compiled
+// one (8, 16, 24, 32; the chain table is that degree's), which writes only
+// its degrees l <= L.  Degree 12 so
+// costs degree 16's arithmetic, 1.7 times its own, and is still far ahead of
+// the runtime-degree kernel above, which reduces over the wave once per
+// degree (FP64, us: 10242 cells degree 12 30.7 -> 6.3, 163842 cells degree 20
+// 81 -> 21).
 constexpr int kPairWaves = 4;
 
 template <int LT>
@@ -1494,13 +1506,15 @@ __device__ __forceinline__ void pair_dispatch(int pair, int N, const double *__r
 }
 
 template <typename T, int LT>
-__global__ __launch_bounds__(64 * kPairWaves) void k_sh_analysis_pair(int N, const double *__restrict__ chain,
+__global__ __launch_bounds__(64 * kPairWaves) void k_sh_analysis_pair(int Lout, int N,
+                                                                      const double *__restrict__ chain,
                                                                       const double *__restrict__ trig,
                                                                       const T *__restrict__ x, long long x_stride,
                                                                       int R, int n_cblk, int n_logical,
                                                                       double *b_part) {
   using S = PairShape<LT>;
-  constexpr int L = LT, K = (L + 1) * (L + 1), n_pairs = L / 2 + 1;
+  constexpr int L = LT, n_pairs = L / 2 + 1;
+  const int K = (Lout + 1) * (Lout + 1);
   constexpr int NTASK = kPairWaves * S::CH * 4;  // (wave, sum, lane group of 16)
   __shared__ double red[kPairWaves * 64 * (S::CH + 1)];
   __shared__ double red2[NTASK];
@@ -1553,7 +1567,7 @@ __global__ __launch_bounds__(64 * kPairWaves) void k_sh_analysis_pair(int N, con
   const int t = v >> 1;
   const bool sn = (v & 1) != 0;
   const int m = t < nA ? m0 : m1, kk = t < nA ? t : t - nA, l = m + kk;
-  if (sn && m == 0) return;
+  if ((sn && m == 0) || l > Lout) return;
   const double scale = chain[2 * ((t < nA ? offA : offB) + kk) + 1];
   b_part[(size_t(b) * n_cblk + cblk) * K + l * l + l + (sn ? -m : m)] = scale * tot[v];
 }
@@ -1590,13 +1604,12 @@ __device__ __forceinline__ T synth_degree(int L, int m, const double *__restrict
   return acc;
 }
 
-template <typename T, int LT>
-__global__ __launch_bounds__(kBlock) void k_sh_synth_rec(int Lrt, int N, const double *__restrict__ tabm,
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_sh_synth_rec(int L, int N, const double *__restrict__ tabm,
                                                          const double *__restrict__ trig,
                                                          const double *__restrict__ cmaj, const T *base,
                                                          long long stride, T *out, int4 mr4) {
   __shared__ double part[kBlock];
-  const int L = LT > 0 ? LT : Lrt;
   const int b = blockIdx.y;
   const double *tsect = tabm, *tf1 = tabm + (L + 1);
   const double *cb = cmaj + size_t(b) * (L + 1) * (L + 2);
@@ -1640,8 +1653,9 @@ __global__ __launch_bounds__(kBlock) void k_sh_synth_rec(int Lrt, int N, const d
   out[b * stride + i] = add + T(sum);
 }
 
-// Synthesis with the rescaled recurrence, for a degree L fixed at compile
-// time: 128 cells x 4 waves per workgroup, each lane two cells (i, i + 64),
+// Synthesis with the rescaled recurrence, for degree LT fixed at compile time
+// (0: any; 21.3 against 18.7 us at degree 32 on 40962 cells): 128 cells x 4
+// waves per workgroup, each lane two cells (i, i + 64),
 // wave g summing the contiguous m-range of synth_split (cos / sin (m lon)
 // by rotation, P_mm = P_{m-1,m-1} sect_m cos(lat)).  Each m sums its
 // degrees against the degree table (beta_l, S_l c_{l,m}, S_l c_{l,-m}, 0)
@@ -1663,13 +1677,12 @@ __device__ __forceinline__ void synth_next_m(SynthCell<T> &c, double sect) {
 }
 
 template <typename T, int LT>
-__global__ __launch_bounds__(kBlock) void k_sh_synth_chain(int N, const double *__restrict__ chain,
-                                                           const double *__restrict__ tabm,
+__global__ __launch_bounds__(kBlock) void k_sh_synth_chain(int Lrt, int N, const double *__restrict__ tabm,
                                                            const double *__restrict__ trig,
                                                            const double *__restrict__ cmaj, const T *base,
                                                            long long stride, T *out, int4 mr4) {
   __shared__ double part[2][kBlock];
-  constexpr int L = LT;
+  const int L = LT > 0 ? LT : Lrt;
   const int b = blockIdx.y;
   const double *cb = cmaj + size_t(b) * 2 * (L + 1) * (L + 2);
   const int lane = threadIdx.x & 63;
@@ -2269,6 +2282,7 @@ struct odis_ctx {
   double *sh_tab = nullptr, *sh_trig = nullptr;  // recurrence table, [4][N] sin/cos lat, cos/sin lon
   double *sh_tabm = nullptr, *sh_cmaj = nullptr; // m-major table, m-major coefficients [B][2 (L+1)(L+2)]
   double *sh_chain = nullptr;                    // rescaled recurrence (beta, S) per (l, m), then C_m
+  double *sh_chain_ana = nullptr;                // the same for the degree of the pair analysis
   uint4 *sh_Ya = nullptr, *sh_Ys = nullptr;      // batched products: split basis in fragment order
   uint4 *sh_Xa = nullptr;                        // batched products: split eta of the batch (analysis operand)
   unsigned short *sh_Cs = nullptr;               // batched products: split coefficients [B][Kp / 32][4][16]
@@ -3219,36 +3233,50 @@ static int stage_coefficients(odis_ctx *ctx, long long n0, int count, const doub
   return ODIS_OK;
 }
 
-// On-the-fly analysis with CPT cells per lane: the degree-32 kernel with its
-// loops unrolled at compile time, or the runtime-degree one.
+// On-the-fly analysis of degrees without a pair kernel, CPT cells per lane.
 template <typename T, int CPT>
 static void launch_analysis_rec(odis_ctx *ctx, int nb, int L, const T *x, long long stride, int n_chunks,
                                 hipEvent_t e0, hipEvent_t e1) {
   const int n_cblk = (n_chunks + kShWaves - 1) / kShWaves;
-  const dim3 ga(n_cblk * (L / 2 + 1), nb), blk(64 * kShWaves);
-  const size_t lds = sizeof(double) * kShWaves * 2 * (L + 2);
-  if (L == 32)
-    hipExtLaunchKernelGGL((k_sh_analysis_rec<T, 32, CPT>), ga, blk, lds, ctx->stream, e0, e1, 0, L, ctx->N,
-                          ctx->sh_tabm, ctx->sh_trig, x, stride, n_chunks, ctx->sh_b);
-  else
-    hipExtLaunchKernelGGL((k_sh_analysis_rec<T, 0, CPT>), ga, blk, lds, ctx->stream, e0, e1, 0, L, ctx->N,
-                          ctx->sh_tabm, ctx->sh_trig, x, stride, n_chunks, ctx->sh_b);
+  const dim3 ga(n_cblk * (L + 1), nb), blk(64 * kShWaves);
+  const size_t lds = sizeof(double) * kShWaves * 2 * (L + 1);
+  hipExtLaunchKernelGGL((k_sh_analysis_rec<T, CPT>), ga, blk, lds, ctx->stream, e0, e1, 0, L, ctx->N, ctx->sh_tabm,
+                        ctx->sh_trig, x, stride, n_chunks, ctx->sh_b);
 }
 
-// Degrees with a compiled pair analysis (the others use the per-degree one).
-static bool pair_degree(int L) { return L == 8 || L == 16 || L == 32; }
+// Degree of the pair analysis that runs degree L (0: none, the per-degree
+// one).  FP64 contexts run a degree up to 32 in the next compiled one; FP32
+// contexts only a compiled degree itself: a stiff shell multiplies the
+// rounding of the FP32 sums by up to 1e4, so their order is left as it is.
+static int pair_degree(const odis_ctx *ctx, int L) {
+  if (ctx->precision == ODIS_FP32) return L == 8 || L == 16 || L == 32 ? L : 0;
+  return L <= 8 ? 8 : (L <= 16 ? 16 : (L <= 24 ? 24 : (L <= 32 ? 32 : 0)));
+}
+
+template <typename T>
+static const void *pair_kernel(int LT) {
+  switch (LT) {
+    case 8: return reinterpret_cast<const void *>(&k_sh_analysis_pair<T, 8>);
+    case 16: return reinterpret_cast<const void *>(&k_sh_analysis_pair<T, 16>);
+    case 24: return reinterpret_cast<const void *>(&k_sh_analysis_pair<T, 24>);
+    default: return reinterpret_cast<const void *>(&k_sh_analysis_pair<T, 32>);
+  }
+}
+
+// Grids too small for one full round still take 4 cells per lane: with 2 the
+// block reductions cost more than the workgroups gain (degree 32 on 10242
+// cells 12.1 against 9.9 us, a degree-16 step on 40962 31.5 against 30.3).
+constexpr int kPairMinCells = 4;
 
 // Cells per lane of the pair analysis when none is set: the grid
 // (ceil(N / (64 kPairWaves R)) cell blocks x pairs x instances) fits the
 // workgroups the device holds at once (one round, no tail), R even and >= 4.
 template <typename T>
-static int pair_auto_cells(odis_ctx *ctx, int L, int nb) {
+static int pair_auto_cells(odis_ctx *ctx, int L, int nb) {  // L: of the kernel
   int per_cu = 0, n_cu = 0, dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e == hipSuccess) e = hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev);
-  const void *k = L == 32 ? reinterpret_cast<const void *>(&k_sh_analysis_pair<T, 32>)
-                          : (L == 16 ? reinterpret_cast<const void *>(&k_sh_analysis_pair<T, 16>)
-                                     : reinterpret_cast<const void *>(&k_sh_analysis_pair<T, 8>));
+  const void *k = pair_kernel<T>(L);
   if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, 64 * kPairWaves, 0);
   if (e != hipSuccess || per_cu <= 0 || n_cu <= 0) return 16;
   const int n_pairs = L / 2 + 1;
@@ -3257,16 +3285,16 @@ static int pair_auto_cells(odis_ctx *ctx, int L, int nb) {
   const long long span = 64LL * kPairWaves * n_cblk;
   int R = int((ctx->N + span - 1) / span);
   R += R & 1;
-  return std::max(4, R);
+  return std::max(kPairMinCells, R);
 }
 
 template <typename T, int LT>
 static void launch_analysis_pair(odis_ctx *ctx, int nb, const T *x, long long stride, int cpt, int n_cblk,
                                  hipEvent_t e0, hipEvent_t e1) {
-  const int n_logical = n_cblk * (LT / 2 + 1);
+  const int n_logical = n_cblk * (LT / 2 + 1);  // degrees above ctx->sh_L are not written
   const dim3 ga((n_logical + 7) / 8 * 8, nb), blk(64 * kPairWaves);
-  hipExtLaunchKernelGGL((k_sh_analysis_pair<T, LT>), ga, blk, 0, ctx->stream, e0, e1, 0, ctx->N, ctx->sh_chain,
-                        ctx->sh_trig, x, stride, cpt, n_cblk, n_logical, ctx->sh_b);
+  hipExtLaunchKernelGGL((k_sh_analysis_pair<T, LT>), ga, blk, 0, ctx->stream, e0, e1, 0, ctx->sh_L, ctx->N,
+                        ctx->sh_chain_ana, ctx->sh_trig, x, stride, cpt, n_cblk, n_logical, ctx->sh_b);
 }
 
 // Batched products: NIT instance tiles per wave (all of the batch up to
@@ -3354,11 +3382,12 @@ static int sh_apply(odis_ctx *ctx, const T *x, long long stride, int nb, const d
   const dim3 blk(kBlock);
   const bool split = ctx->sh_mode == ODIS_SH_SPLIT_BF16;
   // on the fly: chunks of 64 CPT cells, partials per workgroup of kShWaves chunks
-  const bool by_pair = ctx->sh_mode == ODIS_SH_RECUR && pair_degree(L);
+  const int LT = pair_degree(ctx, L);
+  const bool by_pair = ctx->sh_mode == ODIS_SH_RECUR && LT;
   const bool mfma = ctx->sh_mode == ODIS_SH_MFMA;
   // cells per lane: the option, else for the pair analysis the fewest that
   // fit its grid in one round of resident workgroups, 8 for the per-degree one
-  const int cpt = ctx->sh_cpt ? ctx->sh_cpt : (by_pair ? pair_auto_cells<T>(ctx, L, nb) : 8);
+  const int cpt = ctx->sh_cpt ? ctx->sh_cpt : (by_pair ? pair_auto_cells<T>(ctx, LT, nb) : 8);
   const int n_chunks = (N + 64 * cpt - 1) / (64 * cpt);
   // cmaj holds S_l c for the compiled-degree synthesis
   const double *chain = by_pair ? ctx->sh_chain : nullptr;
@@ -3374,9 +3403,11 @@ static int sh_apply(odis_ctx *ctx, const T *x, long long stride, int nb, const d
   } else if (by_pair) {
     if (ana) {
       hipEvent_t e0 = ev ? ev[0] : nullptr, e1 = ev ? ev[1] : nullptr;
-      if (L == 32)
+      if (LT == 32)
         launch_analysis_pair<T, 32>(ctx, nb, x, stride, cpt, n_cblk, e0, e1);
-      else if (L == 16)
+      else if (LT == 24)
+        launch_analysis_pair<T, 24>(ctx, nb, x, stride, cpt, n_cblk, e0, e1);
+      else if (LT == 16)
         launch_analysis_pair<T, 16>(ctx, nb, x, stride, cpt, n_cblk, e0, e1);
       else
         launch_analysis_pair<T, 8>(ctx, nb, x, stride, cpt, n_cblk, e0, e1);
@@ -3422,17 +3453,15 @@ static int sh_apply(odis_ctx *ctx, const T *x, long long stride, int nb, const d
     const dim3 gs((N + 63) / 64, nb), gs2((N + 127) / 128, nb);
     const int4 mr = synth_split(L);
     hipEvent_t e4 = ev ? ev[4] : nullptr, e5 = ev ? ev[5] : nullptr;
-    if (L == 32)
-      hipExtLaunchKernelGGL((k_sh_synth_chain<T, 32>), gs2, blk, 0, ctx->stream, e4, e5, 0, N, ctx->sh_chain,
-                            ctx->sh_tabm, ctx->sh_trig, ctx->sh_cmaj, base, stride, out, mr);
-    else if (L == 16)
-      hipExtLaunchKernelGGL((k_sh_synth_chain<T, 16>), gs2, blk, 0, ctx->stream, e4, e5, 0, N, ctx->sh_chain,
-                            ctx->sh_tabm, ctx->sh_trig, ctx->sh_cmaj, base, stride, out, mr);
-    else if (L == 8)
-      hipExtLaunchKernelGGL((k_sh_synth_chain<T, 8>), gs2, blk, 0, ctx->stream, e4, e5, 0, N, ctx->sh_chain,
-                            ctx->sh_tabm, ctx->sh_trig, ctx->sh_cmaj, base, stride, out, mr);
+    if (by_pair) {
+      auto chain_kernel = L == 32 ? &k_sh_synth_chain<T, 32>
+                                  : (L == 16 ? &k_sh_synth_chain<T, 16>
+                                             : (L == 8 ? &k_sh_synth_chain<T, 8> : &k_sh_synth_chain<T, 0>));
+      hipExtLaunchKernelGGL(chain_kernel, gs2, blk, 0, ctx->stream, e4, e5, 0, L, N, ctx->sh_tabm, ctx->sh_trig,
+                            ctx->sh_cmaj, base, stride, out, mr);
+    }
     else
-      hipExtLaunchKernelGGL((k_sh_synth_rec<T, 0>), gs, blk, 0, ctx->stream, e4, e5, 0, L, N, ctx->sh_tabm,
+      hipExtLaunchKernelGGL((k_sh_synth_rec<T>), gs, blk, 0, ctx->stream, e4, e5, 0, L, N, ctx->sh_tabm,
                             ctx->sh_trig, ctx->sh_cmaj, base, stride, out, mr);
   } else if (syn) {
     const dim3 gs((N + 63) / 64, nb);
@@ -4962,6 +4991,35 @@ static bool spd_inverse(std::vector<double> &A, int n) {
   return true;
 }
 
+// Rescaled chains to degree L: q_l = mu q_{l-1} + beta_l q_{l-2}, P_lm = S_l
+// q_l; per m and l the pair (beta, S), then C_m.
+static void chain_table(int L, std::vector<double> &chain) {
+  std::vector<double> a, bt, sect, f1;
+  odis::sh_recurrence_tables(L, a, bt, sect, f1);
+  for (int m = 0; m <= L; m++) {
+    double S = 1.0, a_prev = f1[m];
+    chain.push_back(1.0);  // k = 0: q = P_mm through q_{-2}
+    chain.push_back(1.0);
+    if (m < L) {
+      S = f1[m];
+      chain.push_back(0.0);  // k = 1: q = mu P_mm
+      chain.push_back(S);
+    }
+    for (int l = m + 2; l <= L; l++) {
+      const double al = a[odis::sh_lm_index(l, m)], bl = bt[odis::sh_lm_index(l, m)];
+      S *= al;
+      chain.push_back(-bl / (al * a_prev));
+      chain.push_back(S);
+      a_prev = al;
+    }
+  }
+  double C = 1.0;
+  for (int m = 0; m <= L; m++) {
+    if (m > 0) C *= sect[m];
+    chain.push_back(C);
+  }
+}
+
 static int sh_set_basis_impl(odis_ctx *ctx, int l_max, const double *beta, int mode) {
   if (!ctx) return ODIS_E_INVALID;
   if (mode != ODIS_SH_OFF && mode != ODIS_SH_FP64 && mode != ODIS_SH_SPLIT_BF16 && mode != ODIS_SH_RECUR &&
@@ -4976,7 +5034,7 @@ static int sh_set_basis_impl(odis_ctx *ctx, int l_max, const double *beta, int m
   ctx->sh_mode = ODIS_SH_OFF;
   ctx->sh_L = ctx->sh_K = 0;
   ctx->sh_Yt = ctx->sh_Minv = ctx->sh_D = ctx->sh_b = ctx->sh_c = ctx->sh_tab = ctx->sh_trig = nullptr;
-  ctx->sh_tabm = ctx->sh_cmaj = ctx->sh_chain = nullptr;
+  ctx->sh_tabm = ctx->sh_cmaj = ctx->sh_chain = ctx->sh_chain_ana = nullptr;
   ctx->sh_Yp = nullptr;
   ctx->sh_Ya = ctx->sh_Ys = ctx->sh_Xa = nullptr;
   ctx->sh_Cs = nullptr;
@@ -5056,32 +5114,15 @@ static int sh_set_basis_impl(odis_ctx *ctx, int l_max, const double *beta, int m
       }
     if ((rc = alloc(reinterpret_cast<void **>(&ctx->sh_tabm), tabm.size() * sizeof(double)))) return rc;
     CK(hipMemcpy(ctx->sh_tabm, tabm.data(), tabm.size() * sizeof(double), hipMemcpyHostToDevice));
-    // rescaled chains: q_l = mu q_{l-1} + beta_l q_{l-2}, P_lm = S_l q_l
-    std::vector<double> chain;
-    for (int m = 0; m <= l_max; m++) {
-      double S = 1.0, a_prev = f1[m];
-      chain.push_back(1.0);  // k = 0: q = P_mm through q_{-2}
-      chain.push_back(1.0);
-      if (m < l_max) {
-        S = f1[m];
-        chain.push_back(0.0);  // k = 1: q = mu P_mm
-        chain.push_back(S);
-      }
-      for (int l = m + 2; l <= l_max; l++) {
-        const double al = a[odis::sh_lm_index(l, m)], bl = bt[odis::sh_lm_index(l, m)];
-        S *= al;
-        chain.push_back(-bl / (al * a_prev));
-        chain.push_back(S);
-        a_prev = al;
-      }
-    }
-    double C = 1.0;
-    for (int m = 0; m <= l_max; m++) {
-      if (m > 0) C *= sect[m];
-      chain.push_back(C);
-    }
+    std::vector<double> chain, chain_ana;
+    chain_table(l_max, chain);
     if ((rc = alloc(reinterpret_cast<void **>(&ctx->sh_chain), chain.size() * sizeof(double)))) return rc;
     CK(hipMemcpy(ctx->sh_chain, chain.data(), chain.size() * sizeof(double), hipMemcpyHostToDevice));
+    if (const int LT = pair_degree(ctx, l_max)) {
+      chain_table(LT, chain_ana);
+      if ((rc = alloc(reinterpret_cast<void **>(&ctx->sh_chain_ana), chain_ana.size() * sizeof(double)))) return rc;
+      CK(hipMemcpy(ctx->sh_chain_ana, chain_ana.data(), chain_ana.size() * sizeof(double), hipMemcpyHostToDevice));
+    }
     // coefficients: pairs (runtime degrees) or the 4-double degree table of
     // the chain synthesis, with beta and the padding set here
     const size_t nlm = size_t(l_max + 1) * (l_max + 2) / 2;
@@ -5095,9 +5136,9 @@ static int sh_set_basis_impl(odis_ctx *ctx, int l_max, const double *beta, int m
     }
     if ((rc = alloc(reinterpret_cast<void **>(&ctx->sh_trig), trig.size() * sizeof(double)))) return rc;
     CK(hipMemcpy(ctx->sh_trig, trig.data(), trig.size() * sizeof(double), hipMemcpyHostToDevice));
-    // the most partials: 4 cells per lane
+    // the most partials: the fewest cells per lane
     ctx->sh_part = std::max(((N + 64 * 4 - 1) / (64 * 4) + kShWaves - 1) / kShWaves,
-                            (N + 64 * kPairWaves * 4 - 1) / (64 * kPairWaves * 4));
+                            (N + 64 * kPairWaves * kPairMinCells - 1) / (64 * kPairWaves * kPairMinCells));
   }
   if (mode == ODIS_SH_MFMA) {
     // the FP64 basis was only needed for the Gram matrix

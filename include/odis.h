@@ -276,10 +276,10 @@ int odis_request_stop(odis_ctx *ctx);
  *  ODIS_OPT_STEP_LANES lanes per cell of the one-kernel step: 4 (default,
  *                    about one face per lane) or 2 (about two).
  *  ODIS_OPT_SH_CELLS cells per lane of the on-the-fly SH analysis: 0
- *                    (default: for degrees 8, 16 and 32, which have
- *                    compiled kernels, the fewest even count >= 4 whose grid
- *                    fits the workgroups the device holds at once; 8 for the
- *                    others), 4, 8 or 16; the coefficients depend on it by
+ *                    (default: for degrees 8, 16 and 32, in FP64 up to
+ *                    32, which have compiled kernels, the fewest even count
+ *                    >= 4 whose grid fits the workgroups the device holds at
+ *                    once; 8 for the others), 4, 8 or 16; the coefficients depend on it by
  *                    rounding only.
  *  ODIS_OPT_INTERLEAVE a batch steps with its state held interleaved
  *                    (groups of 16 instances, instances innermost), one
