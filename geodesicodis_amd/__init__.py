@@ -502,7 +502,7 @@ class Context:
 
     def sh_synthesize(self, coeffs):
         c = np.ascontiguousarray(coeffs, np.float64)
-        f = np.zeros(self.mesh.N)
+        f = np.empty(self.mesh.N)
         self._check(lib().odis_sh_synthesize(self._h, _dp(c), _dp(f)))
         return f
 
