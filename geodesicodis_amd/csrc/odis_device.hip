@@ -1021,12 +1021,25 @@ __global__ __launch_bounds__(kBlock) void k_sh_analysis(int K, int N, const doub
   if (threadIdx.x == 0) b_part[(size_t(b) * kShChunks + q) * K + k] = t;
 }
 
+// The chains of the degree table are padded to whole groups of kChainGroup
+// degrees: chain_at is where order m starts, chain_at(L, L + 1) the size.
+constexpr int kChainGroup = 4;
+
+__host__ __device__ constexpr int chain_groups(int n) {  // sum of ceil(j / kChainGroup) for j = 1 .. n
+  const int q = n / kChainGroup, r = n % kChainGroup;
+  return kChainGroup * q * (q + 1) / 2 + r * (q + 1);
+}
+
+__host__ __device__ constexpr int chain_at(int L, int m) {
+  return kChainGroup * (chain_groups(L + 1) - chain_groups(L + 1 - m));
+}
+
 // Store c_k (k = l l + l + m) at its m-major place: for m = 0..L, l = m..L
 // the pair (c_{l,|m|}, c_{l,-|m|}) at 2 (m (L + 1) - m (m - 1) / 2 + l - m);
 // the unused sine slot of m = 0 is zero.  chain (nullable): the degree
-// table of the chain synthesis instead, 4 doubles per (l, m) at
-// 4 (m (L + 1) - m (m - 1) / 2 + l - m): (beta_l, S_l c_{l,m}, S_l c_{l,-m}, 0),
-// S_l the chain scale; beta and the padding are set with the basis.
+// table of the chain synthesis instead, 3 doubles per (l, m) at
+// 3 (chain_at(L, m) + l - m): (beta_l, S_l c_{l,m}, S_l c_{l,-m}), S_l the
+// chain scale; beta and the padding are set with the basis.
 __device__ __forceinline__ void put_mmajor(int K, int b, int k, double ck, const double *chain, double *cmaj) {
   int l = 0;
   while ((l + 1) * (l + 1) <= k) ++l;
@@ -1035,9 +1048,9 @@ __device__ __forceinline__ void put_mmajor(int K, int b, int k, double ck, const
   while ((L + 1) * (L + 1) < K) ++L;
   const int at = m * (L + 1) - m * (m - 1) / 2 + l - m;
   if (chain) {
-    double *cb = cmaj + size_t(b) * 2 * (L + 1) * (L + 2);
-    if (m == 0) cb[4 * at + 2] = 0.0;
-    cb[4 * at + 1 + (mm < 0 ? 1 : 0)] = chain[2 * at + 1] * ck;
+    double *cb = cmaj + size_t(b) * 3 * chain_at(L, L + 1) + 3 * (chain_at(L, m) + l - m);
+    if (m == 0) cb[2] = 0.0;
+    cb[mm < 0 ? 2 : 1] = chain[2 * at + 1] * ck;
   } else {
     double *cb = cmaj + size_t(b) * (L + 1) * (L + 2);
     if (m == 0) cb[2 * l + 1] = 0.0;
@@ -1653,16 +1666,27 @@ __global__ __launch_bounds__(kBlock) void k_sh_synth_rec(int L, int N, const dou
   out[b * stride + i] = add + T(sum);
 }
 
-// Synthesis with the rescaled recurrence, for degree LT fixed at compile time
-// (0: any; 21.3 against 18.7 us at degree 32 on 40962 cells): 128 cells x 4
-// waves per workgroup, each lane two cells (i, i + 64),
-// wave g summing the contiguous m-range of synth_split (cos / sin (m lon)
-// by rotation, P_mm = P_{m-1,m-1} sect_m cos(lat)).  Each m sums its
-// degrees against the degree table (beta_l, S_l c_{l,m}, S_l c_{l,-m}, 0)
-// written by put_mmajor, four operations per degree and cell:
+// Synthesis with the rescaled recurrence: 128 cells x NW waves per
+// workgroup, each lane two cells (i, i + 64), wave g summing the orders
+// [cut[g], cut[g + 1]).  Each m sums its degrees against the degree table
+// (beta_l, S_l c_{l,m}, S_l c_{l,-m}) written by put_mmajor, four operations
+// per degree and cell:
 //     q_l = mu q_{l-1} + beta_l q_{l-2},  A += (S c)_{l,m} q_l,  B += (S c)_{l,-m} q_l,
-// and y = sum_m A_m cos(m lon) + B_m sin(m lon); the four waves' sums are
-// added through LDS in a fixed order.
+// from q_{m-1} = 0, q_{m-2} = P_mm (beta_m = 1, beta_{m+1} = 0), and
+// y = sum_m A_m cos(m lon) + B_m sin(m lon); the waves' sums are added
+// through LDS in a fixed order.
+// A chain is padded with zero entries to whole groups, so a group is one
+// straight run of 32 FP64 operations on one batch of scalar loads, and the
+// first two degrees need no code of their own.  Entries of 24 bytes keep the
+// degree-32 table (14.7 KB) inside the 16 KB scalar cache.  What bounds it:
+// on large grids FP64 issue (163842 cells, degree 32: 64 % of the cycles a CU
+// is busy; 24.3 -> 22.4 us); on small ones the scalar loads, since a
+// workgroup reads every entry once and so mostly misses: more waves share
+// them (degree 32 on 40962 cells 19.9 -> 11.0 us, 16 on 10242 7.8 -> 4.7).
+struct SynthCuts {
+  int m[9];
+};
+
 template <typename T>
 struct SynthCell {
   T mu, s, cl, sl, cm, sm, pmm, y;
@@ -1676,20 +1700,36 @@ __device__ __forceinline__ void synth_next_m(SynthCell<T> &c, double sect) {
   c.pmm = c.pmm * (T(sect) * c.s);
 }
 
-template <typename T, int LT>
-__global__ __launch_bounds__(kBlock) void k_sh_synth_chain(int Lrt, int N, const double *__restrict__ tabm,
-                                                           const double *__restrict__ trig,
-                                                           const double *__restrict__ cmaj, const T *base,
-                                                           long long stride, T *out, int4 mr4) {
-  __shared__ double part[2][kBlock];
-  const int L = LT > 0 ? LT : Lrt;
+// (cos m lon, sin m lon, P_mm = C_m cos^m lat) by binary powers
+template <typename T>
+__device__ __forceinline__ void synth_start(SynthCell<T> &c, int m, double cmm) {
+  T zc = c.cl, zs = c.sl, zr = c.s;
+  for (int k = m; k > 0; k >>= 1) {
+    if (k & 1) {
+      cmul(c.cm, c.sm, zc, zs);
+      c.pmm *= zr;
+    }
+    const T c2 = fma(zc, zc, -(zs * zs));
+    zs = T(2) * (zc * zs);
+    zc = c2;
+    zr *= zr;
+  }
+  c.pmm *= T(cmm);
+}
+
+template <typename T, int NW>
+__global__ __launch_bounds__(64 * NW) void k_sh_synth_chain(int L, int N, const double *__restrict__ sect,
+                                                            const double *__restrict__ chain,
+                                                            const double *__restrict__ trig,
+                                                            const double *__restrict__ cmaj, const T *base,
+                                                            long long stride, T *out, SynthCuts cut) {
+  constexpr int G = kChainGroup;
+  __shared__ double part[2][64 * NW];
   const int b = blockIdx.y;
-  const double *cb = cmaj + size_t(b) * 2 * (L + 1) * (L + 2);
   const int lane = threadIdx.x & 63;
   const int g = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int i0 = blockIdx.x * 128 + lane;
-  const int mlo = g == 0 ? 0 : (g == 1 ? mr4.x : (g == 2 ? mr4.y : mr4.z));
-  const int mhi = g == 0 ? mr4.x : (g == 1 ? mr4.y : (g == 2 ? mr4.z : mr4.w));
+  const int mlo = cut.m[g], mhi = cut.m[g + 1];
   SynthCell<T> u[2];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
@@ -1703,48 +1743,56 @@ __global__ __launch_bounds__(kBlock) void k_sh_synth_chain(int Lrt, int N, const
     u[h].pmm = T(1);
     u[h].y = T(0);
   }
-  for (int q = 1; q < mlo; ++q) {  // advance to m = mlo - 1
-    synth_next_m(u[0], tabm[q]);
-    synth_next_m(u[1], tabm[q]);
-  }
+  if (mlo < mhi) {
+    const double *e = cmaj + size_t(b) * 3 * chain_at(L, L + 1) + 3 * chain_at(L, mlo);
+    if constexpr (sizeof(T) == 8) {
+      const double cmm = chain[(L + 1) * (L + 2) + mlo];
+      synth_start(u[0], mlo, cmm);
+      synth_start(u[1], mlo, cmm);
+    } else {
+      for (int q = 1; q <= mlo; ++q) {
+        synth_next_m(u[0], sect[q]);
+        synth_next_m(u[1], sect[q]);
+      }
+    }
+    T A0 = T(0), B0 = T(0), A1 = T(0), B1 = T(0);
+    T p1 = T(0), p2 = u[0].pmm, r1 = T(0), r2 = u[1].pmm;
+    int m = mlo, left = (L - m + G) / G;
+    double sect_next = sect[min(m + 1, L)];
+    const int total = chain_groups(L + 1 - mlo) - chain_groups(L + 1 - mhi);
 #pragma unroll 1
-  for (int m = mlo; m < mhi; ++m) {
-    if (m > 0) {
-      synth_next_m(u[0], tabm[m]);
-      synth_next_m(u[1], tabm[m]);
+    for (int q = 0; q < total; ++q, e += 3 * G) {
+      double cur[3 * G];
+#pragma unroll
+      for (int k = 0; k < 3 * G; ++k) cur[k] = e[k];
+#pragma unroll
+      for (int k = 0; k < G; ++k) {
+        const T be = T(cur[3 * k]), cc = T(cur[3 * k + 1]), ss = T(cur[3 * k + 2]);
+        const T p = fma(u[0].mu, p1, be * p2);
+        const T r = fma(u[1].mu, r1, be * r2);
+        p2 = p1;
+        p1 = p;
+        r2 = r1;
+        r1 = r;
+        A0 = fma(cc, p, A0);
+        B0 = fma(ss, p, B0);
+        A1 = fma(cc, r, A1);
+        B1 = fma(ss, r, B1);
+      }
+      if (--left == 0) {
+        u[0].y = fma(B0, u[0].sm, fma(A0, u[0].cm, u[0].y));
+        u[1].y = fma(B1, u[1].sm, fma(A1, u[1].cm, u[1].y));
+        synth_next_m(u[0], sect_next);
+        synth_next_m(u[1], sect_next);
+        ++m;
+        left = (L - m + G) / G;
+        sect_next = sect[min(m + 1, L)];
+        A0 = B0 = A1 = B1 = T(0);
+        p1 = r1 = T(0);
+        p2 = u[0].pmm;
+        r2 = u[1].pmm;
+      }
     }
-    const int off = m * (L + 1) - m * (m - 1) / 2, nk = L - m + 1;
-    const double *e = cb + 4 * off;  // (beta, S c, S s, 0) per degree
-    // degrees m and m + 1, then the recurrence (the sine slots of m = 0 are zero)
-    const T c0 = T(e[1]), s0 = T(e[2]);
-    T A0 = c0 * u[0].pmm, B0 = s0 * u[0].pmm, A1 = c0 * u[1].pmm, B1 = s0 * u[1].pmm;
-    T p2 = u[0].pmm, p1 = u[0].pmm, r2 = u[1].pmm, r1 = u[1].pmm;
-    if (nk > 1) {
-      const T c1 = T(e[5]), s1 = T(e[6]);
-      p1 = u[0].mu * p2;
-      r1 = u[1].mu * r2;
-      A0 = fma(c1, p1, A0);
-      B0 = fma(s1, p1, B0);
-      A1 = fma(c1, r1, A1);
-      B1 = fma(s1, r1, B1);
-    }
-    e += 8;
-#pragma unroll 4
-    for (int k = 2; k < nk; ++k, e += 4) {
-      const T be = T(e[0]), cc = T(e[1]), ss = T(e[2]);
-      const T p = fma(u[0].mu, p1, be * p2);
-      const T r = fma(u[1].mu, r1, be * r2);
-      p2 = p1;
-      p1 = p;
-      r2 = r1;
-      r1 = r;
-      A0 = fma(cc, p, A0);
-      B0 = fma(ss, p, B0);
-      A1 = fma(cc, r, A1);
-      B1 = fma(ss, r, B1);
-    }
-    u[0].y = fma(B0, u[0].sm, fma(A0, u[0].cm, u[0].y));
-    u[1].y = fma(B1, u[1].sm, fma(A1, u[1].cm, u[1].y));
   }
   part[0][threadIdx.x] = double(u[0].y);
   part[1][threadIdx.x] = double(u[1].y);
@@ -1752,10 +1800,36 @@ __global__ __launch_bounds__(kBlock) void k_sh_synth_chain(int Lrt, int N, const
   if (threadIdx.x >= 128) return;
   const int h = threadIdx.x >> 6, i = i0 + 64 * h;
   if (i >= N) return;
-  const double *pp = part[h];
-  const double sum = (pp[lane] + pp[64 + lane]) + (pp[128 + lane] + pp[192 + lane]);
+  const double *pp = part[h] + lane;
+  double sum = (pp[0] + pp[64]) + (pp[128] + pp[192]);
+  if constexpr (NW == 8) sum += (pp[256] + pp[320]) + (pp[384] + pp[448]);
   const T add = base ? base[b * stride + i] : T(0);
   out[b * stride + i] = add + T(sum);
+}
+
+// FP64 launches of fewer workgroups (three per CU) at degrees above 8 run
+// eight waves each, others four.  Eight against four, us: degree 32, 321
+// workgroups 11.0 / 16.6, 642 14.7 / 17.4, 963 17.5 / 18.8, 1284 23.8 / 23.1;
+// degree 16, 81 4.7 / 6.3, 642 7.0 / 7.2, 963 8.7 / 8.2, 1284 11.1 / 9.6;
+// degree 8, 642 4.8 / 4.3 (nine orders do not fill eight waves).
+constexpr unsigned int kSynthWideBelow = 768;
+
+// Orders of the NW waves of the chain synthesis: near-equal costs, order m
+// costing its groups plus kChainTurn degrees' worth for the turn to m + 1.
+constexpr int kChainTurn = 3;
+
+static SynthCuts chain_split(int L, int NW) {
+  auto cost = [&](int m) { return (L - m + kChainGroup) / kChainGroup * kChainGroup + kChainTurn; };
+  int total = 0, acc = 0, g = 0;
+  for (int m = 0; m <= L; ++m) total += cost(m);
+  SynthCuts c{};
+  for (int m = 0; m <= L; ++m) {
+    // order m goes to the wave that holds its middle
+    while (g + 1 < NW && (2 * acc + cost(m)) * NW >= 2 * total * (g + 1)) c.m[++g] = m;
+    acc += cost(m);
+  }
+  while (g < NW) c.m[++g] = L + 1;
+  return c;
 }
 
 // Degree ranges of the 4 synthesis waves of a workgroup: near-equal numbers of
@@ -3455,11 +3529,12 @@ static int sh_apply(odis_ctx *ctx, const T *x, long long stride, int nb, const d
     const int4 mr = synth_split(L);
     hipEvent_t e4 = ev ? ev[4] : nullptr, e5 = ev ? ev[5] : nullptr;
     if (by_pair) {
-      auto chain_kernel = L == 32 ? &k_sh_synth_chain<T, 32>
-                                  : (L == 16 ? &k_sh_synth_chain<T, 16>
-                                             : (L == 8 ? &k_sh_synth_chain<T, 8> : &k_sh_synth_chain<T, 0>));
-      hipExtLaunchKernelGGL(chain_kernel, gs2, blk, 0, ctx->stream, e4, e5, 0, L, N, ctx->sh_tabm, ctx->sh_trig,
-                            ctx->sh_cmaj, base, stride, out, mr);
+      // FP32 contexts keep the order of their sums (see pair_degree)
+      const bool wide = sizeof(T) == 8 && L > 8 && gs2.x * nb < kSynthWideBelow;
+      const SynthCuts cut = sizeof(T) == 8 ? chain_split(L, wide ? 8 : 4) : SynthCuts{{0, mr.x, mr.y, mr.z, mr.w}};
+      hipExtLaunchKernelGGL((wide ? &k_sh_synth_chain<T, 8> : &k_sh_synth_chain<T, 4>), gs2, dim3(wide ? 512 : 256),
+                            0, ctx->stream, e4, e5, 0, L, N, ctx->sh_tabm, ctx->sh_chain, ctx->sh_trig, ctx->sh_cmaj,
+                            base, stride, out, cut);
     }
     else
       hipExtLaunchKernelGGL((k_sh_synth_rec<T>), gs, blk, 0, ctx->stream, e4, e5, 0, L, N, ctx->sh_tabm,
@@ -5125,15 +5200,15 @@ static int sh_set_basis_impl(odis_ctx *ctx, int l_max, const double *beta, int m
       if ((rc = alloc(reinterpret_cast<void **>(&ctx->sh_chain_ana), chain_ana.size() * sizeof(double)))) return rc;
       CK(hipMemcpy(ctx->sh_chain_ana, chain_ana.data(), chain_ana.size() * sizeof(double), hipMemcpyHostToDevice));
     }
-    // coefficients: pairs (runtime degrees) or the 4-double degree table of
+    // coefficients: pairs (runtime degrees, smaller) or the degree table of
     // the chain synthesis, with beta and the padding set here
-    const size_t nlm = size_t(l_max + 1) * (l_max + 2) / 2;
-    if ((rc = alloc(reinterpret_cast<void **>(&ctx->sh_cmaj), size_t(ctx->B) * 4 * nlm * sizeof(double))))
-      return rc;
+    const size_t ct_one = size_t(3) * chain_at(l_max, l_max + 1), ct_all = ctx->B * ct_one;
+    if ((rc = alloc(reinterpret_cast<void **>(&ctx->sh_cmaj), ct_all * sizeof(double)))) return rc;
     {
-      std::vector<double> ct(size_t(ctx->B) * 4 * nlm, 0.0);
+      std::vector<double> ct(ct_all, 0.0);
       for (int b = 0; b < ctx->B; b++)
-        for (size_t q = 0; q < nlm; q++) ct[(size_t(b) * nlm + q) * 4] = chain[2 * q];
+        for (int m = 0, q = 0; m <= l_max; m++)
+          for (int l = m; l <= l_max; l++, q++) ct[b * ct_one + 3 * (chain_at(l_max, m) + l - m)] = chain[2 * q];
       CK(hipMemcpy(ctx->sh_cmaj, ct.data(), ct.size() * sizeof(double), hipMemcpyHostToDevice));
     }
     if ((rc = alloc(reinterpret_cast<void **>(&ctx->sh_trig), trig.size() * sizeof(double)))) return rc;

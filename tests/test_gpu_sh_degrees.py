@@ -46,3 +46,24 @@ def test_coupled_step_in_the_next_degrees_kernel(product, oracle, precision, lev
     tol = 1e-10 if precision == 0 else 1e-4
     for k in ("v", "eta", "dvdt"):
         assert rel_l2(out[0][k], out[1][k]) < tol, k
+
+
+@pytest.mark.parametrize("level,n_many,degree", [(4, 130, 9), (4, 130, 15), (4, 130, 16), (5, 40, 24), (5, 40, 31),
+                                                 (5, 40, 32)])
+def test_coupled_step_of_many_and_one(product, level, n_many, degree):
+    """A batch large enough for four synthesis waves per workgroup against
+    one instance, which runs eight: the same sums in another order, 20 steps."""
+    G = product
+    g, _ = generated_grid(level)
+    mesh = G.Mesh(g, 232.1e3)
+    beta = G.surface_beta(G.LID_MEMBR, degree, 252.1e3, 0.113, 5e3, 38e3)
+    p, _ = G.make_params(radius=232.1e3, g=0.1166, surface=G.LID_MEMBR, shell_thickness=5e3, time_step=2.0)
+    out = []
+    for n in (1, n_many):  # 6 and 780, 21 and 840 workgroups
+        c = G.Context(mesh, [p] * n)
+        c.set_sh(degree, beta, mode=G.SH_RECUR)
+        c.step(20)
+        out.append(c.get_state(n - 1))
+        c.close()
+    for k in ("v", "eta", "dvdt"):
+        assert rel_l2(out[1][k], out[0][k]) < 1e-10, k
