@@ -293,8 +293,8 @@ int odis_request_stop(odis_ctx *ctx);
  *                    to date when the state is read or set.  The state is the
  *                    same bit for bit; dissipation sums differ by rounding
  *                    (another grouping of the per-face terms).
- *  ODIS_OPT_INTERLEAVE_ACTIVE (read only) 1 when the next step would run
- *                    interleaved.
+ *  ODIS_OPT_INTERLEAVE_ACTIVE (read only) 1 when a step launched by itself
+ *                    would run interleaved (longer runs may run resident).
  *  ODIS_OPT_IL_UNROLL faces and (cell, instance) pairs each lane of the
  *                    interleaved step keeps in flight: 0 (default: 4 and 2
  *                    in FP64, 2 and 1 in FP32), 1 (1, 1), 2 (2, 1), 3 (4, 2).
