@@ -4308,12 +4308,45 @@ static int launch_resident(odis_ctx *ctx, Ops<T> &o, const double *table, int co
   return ODIS_OK;
 }
 
+// The state in the layout (interleaved or instance-major) of the step launches
+// that follow.
 template <typename T>
-static int step_t(odis_ctx *ctx, Ops<T> &o, int n_steps);
+static int enter_layout(odis_ctx *ctx, Ops<T> &o, bool il) {
+  int rc;
+  if (il) {
+    if (!ctx->il_fresh) {  // the instance-major arrays are current: copy them in
+      if ((rc = ensure_ts(ctx, o)) || (rc = il_alloc<T>(ctx)) || (rc = il_convert(ctx, o, true))) return rc;
+      ctx->il_fresh = 1;
+    }
+    if ((rc = il_records(ctx, o))) return rc;
+    ctx->std_fresh = 0;
+  } else {
+    if ((rc = il_out(ctx, o)) || (rc = ensure_ts(ctx, o))) return rc;
+    ctx->il_fresh = 0;
+  }
+  return ODIS_OK;
+}
+
+// n_steps steps with a launch each, for steps a taken-back launch owes: they
+// were accepted earlier, so a stop requested since does not end them, and no
+// kernel of theirs is sampled.
+template <typename T>
+static int step_again(odis_ctx *ctx, Ops<T> &o, long long n_steps) {
+  int rc = enter_layout(ctx, o, il_wanted(ctx));
+  while (!rc && n_steps > 0) {
+    const int count = int(std::min<long long>(ctx->chunk, n_steps));
+    const double *table = nullptr;
+    if ((rc = stage_coefficients(ctx, ctx->step, count, &table))) break;
+    if ((rc = launch_chunk(ctx, o, table, count, nullptr, nullptr))) break;
+    ctx->step += count;
+    n_steps -= count;
+  }
+  return rc;
+}
 
 // Wait for the resident launches enqueued so far and learn whether they ran.
-// Steps of a launch that was taken back (nothing of it, nor of the later
-// ones, was written) are stepped again with a launch each.  Called before
+// The steps of a launch that was taken back and of all later ones (nothing of
+// them was written) are stepped again with a launch each.  Called before
 // anything reads the state or steps by another kernel.
 static int res_settle(odis_ctx *ctx) {
   ResDev &r = ctx->res;
@@ -4326,11 +4359,11 @@ static int res_settle(odis_ctx *ctx) {
   r.off = 1;
   if (st == kResFailed) return fail(ctx, ODIS_E_HIP, "resident step: a workgroup did not answer in time");
   for (const auto &p : sent)
-    if (p.launch == st) {
+    if (p.launch >= st) {
       const long long n = ctx->step - p.n0;
       ctx->step = p.n0;
       ctx->cur = p.cur;
-      return ctx->precision == ODIS_FP64 ? step_t(ctx, ctx->d, int(n)) : step_t(ctx, ctx->f, int(n));
+      return ctx->precision == ODIS_FP64 ? step_again(ctx, ctx->d, n) : step_again(ctx, ctx->f, n);
     }
   return fail(ctx, ODIS_E_HIP, "resident step: unknown launch taken back");
 }
@@ -4346,27 +4379,9 @@ static int step_t(odis_ctx *ctx, Ops<T> &o, int n_steps) {
   std::vector<ChunkEvents> sampled;
   size_t ev_used = 0;
   int done = 0;
-  // the state in the layout of the step launches of the next stretch
-  auto enter = [&](bool il) -> int {
-    if (il) {
-      if (!ctx->il_fresh) {  // the instance-major arrays are current: copy them in
-        int e;
-        if ((e = ensure_ts(ctx, o)) || (e = il_alloc<T>(ctx)) || (e = il_convert(ctx, o, true))) return e;
-        ctx->il_fresh = 1;
-      }
-      const int e = il_records(ctx, o);
-      if (e) return e;
-      ctx->std_fresh = 0;
-    } else {
-      int e;
-      if ((e = il_out(ctx, o)) || (e = ensure_ts(ctx, o))) return e;
-      ctx->il_fresh = 0;
-    }
-    return ODIS_OK;
-  };
   if (res_wanted(ctx) && n_steps >= kResMinSteps && (rc = res_setup<T>(ctx))) return rc;
-  const bool resident = res_wanted(ctx) && n_steps >= kResMinSteps;
-  if (!resident && ((rc = res_settle(ctx)) || (rc = enter(il_wanted(ctx))))) return rc;
+  bool resident = res_wanted(ctx) && n_steps >= kResMinSteps;
+  if (!resident && ((rc = res_settle(ctx)) || (rc = enter_layout(ctx, o, il_wanted(ctx))))) return rc;
   while (done < n_steps) {
     if (ctx->stop_flag) {
       ctx->stop_flag = 0;
@@ -4382,7 +4397,7 @@ static int step_t(odis_ctx *ctx, Ops<T> &o, int n_steps) {
         run = (run + parts - 1) / parts;
       }
       if (run >= kResMinSteps) {
-        if ((rc = enter(false))) return rc;
+        if ((rc = enter_layout(ctx, o, false))) return rc;
         const double *table = nullptr;
         if ((rc = stage_coefficients(ctx, ctx->step, run, &table))) return rc;
         if ((rc = launch_resident(ctx, o, table, run))) return rc;
@@ -4390,7 +4405,8 @@ static int step_t(odis_ctx *ctx, Ops<T> &o, int n_steps) {
         done += run;
         continue;
       }
-      if ((rc = res_settle(ctx)) || (rc = enter(il_wanted(ctx)))) return rc;
+      if ((rc = res_settle(ctx)) || (rc = enter_layout(ctx, o, il_wanted(ctx)))) return rc;
+      resident = res_wanted(ctx);  // not after a launch that was taken back
     }
     const bool graph_fits = ctx->use_graphs && left >= ctx->graph_steps;
     int count = graph_fits ? ctx->graph_steps : std::min(ctx->chunk, left);

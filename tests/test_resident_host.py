@@ -1,0 +1,91 @@
+"""Host logic of the resident step without a GPU: the library runs on a stub
+of the HIP runtime (hip_stub.cpp) in a process of its own.  The stub's kernels
+compute nothing; what is checked is which launches are made, what an entry
+point returns, and what it holds."""
+import os
+import shutil
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+from conftest import ROOT
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+PRELUDE = """
+import ctypes, sys
+S = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+S.stub_log.restype = ctypes.c_char_p
+S.stub_device_bytes.restype = ctypes.c_size_t
+S.stub_fail_allocations_from.argtypes = [ctypes.c_size_t]
+S.stub_end_resident.argtypes = [ctypes.c_int, ctypes.c_uint]
+import numpy as np
+import geodesicodis_amd as G
+
+def log():
+    out = S.stub_log().decode().split("\\n")[:-1]
+    S.stub_clear()
+    return out
+
+def steps(lines, kind="step"):
+    return [int(x.split()[1]) for x in lines if x.startswith(kind + " ")]
+
+def runs(lines):
+    return sum(x.startswith("resident ") for x in lines)
+
+def mesh(level=4):
+    return G.Mesh(G.Grid.generate(level, 64), 252.1e3)
+
+def ocean(n=1, level=4, precision=0, **kw):
+    p = G.make_params(time_step=1.0, **kw)[0]
+    return G.Context(mesh(level), [p] * n, precision=precision)
+
+def refused(call):
+    try:
+        call()
+    except G.OdisError as e:
+        return e.code
+    return 0
+"""
+
+
+@pytest.fixture(scope="module")
+def stub(tmp_path_factory):
+    if not shutil.which("g++"):
+        pytest.skip("no g++")
+    so = tmp_path_factory.mktemp("stub") / "hip_stub.so"
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    os.path.join(HERE, "hip_stub.cpp"), "-o", str(so)], check=True)
+
+    def run(body):
+        r = subprocess.run([sys.executable, "-c", PRELUDE + textwrap.dedent(body), str(so)], cwd=ROOT, timeout=120,
+                           capture_output=True, text=True)
+        assert r.returncode == 0, r.stdout + r.stderr
+    return run
+
+
+@pytest.mark.parametrize("stride", [0, 16])
+def test_steps_of_a_launch_taken_back_are_stepped_once_each(stub, stride):
+    """The first launch, or the second of a timed run, is taken back: every
+    step from there on is launched singly, once, and the call goes on so."""
+    stub("""
+    c = ocean()
+    if %d:
+        c.enable_timing(%d)
+    c.step(1)          # a first single step, then runs
+    log()
+    S.stub_end_resident(%d, 0)
+    c.step(100)
+    lines = log()
+    got = steps(lines)
+    assert c.get_state()["iter"] == 101
+    if %d:   # steps 1..15 in a launch; 16 by itself; the launch of 17..31 is the one taken back
+        assert runs(lines) == 2 and got == list(range(16, 17)) + list(range(17, 101)), lines
+        assert c.timing()["step_ms"] > 0
+    else:
+        assert runs(lines) == 1 and got == list(range(1, 101)), lines
+    c.step(50)         # the context stays on single launches
+    lines = log()
+    assert runs(lines) == 0 and steps(lines) == list(range(101, 151))
+    """ % (stride, stride, 2 if stride else 1, stride))
