@@ -2310,6 +2310,7 @@ struct odis_ctx {
   // resident launches (many steps per launch, odis_resident.hpp)
   int res_opt = 1;             // ODIS_OPT_RESIDENT: 0 off, 1 automatic, > 1 that many patches per instance
   ResDev res;
+  int res_failed = 0;          // a resident launch ended partway: the state is lost
   std::string one_kernel_why;
   std::vector<int> gi_host, cyc_host;  // device-order face cells and cell cycles, to rebuild patches
   std::vector<float> cell_xyz;         // [N][3] unit vectors of the device cells, for the resident patches
@@ -4347,9 +4348,15 @@ static int step_again(odis_ctx *ctx, Ops<T> &o, long long n_steps) {
 // Wait for the resident launches enqueued so far and learn whether they ran.
 // The steps of a launch that was taken back and of all later ones (nothing of
 // them was written) are stepped again with a launch each.  Called before
-// anything reads the state or steps by another kernel.
+// anything reads the state or steps by another kernel.  After a launch that
+// ended partway it fails for good: the histories are updated in place, so
+// there is no state to go back to.
+static int res_failed(odis_ctx *ctx) {
+  return fail(ctx, ODIS_E_HIP, "resident step: a workgroup did not answer in time; the state is lost");
+}
 static int res_settle(odis_ctx *ctx) {
   ResDev &r = ctx->res;
+  if (ctx->res_failed) return res_failed(ctx);
   if (r.pending.empty()) return ODIS_OK;
   CK(hipStreamSynchronize(ctx->stream));
   const std::vector<ResDev::Pending> sent = std::move(r.pending);
@@ -4357,15 +4364,15 @@ static int res_settle(odis_ctx *ctx) {
   const unsigned st = *static_cast<volatile unsigned *>(r.status);
   if (st == 0) return ODIS_OK;
   r.off = 1;
-  if (st == kResFailed) return fail(ctx, ODIS_E_HIP, "resident step: a workgroup did not answer in time");
   for (const auto &p : sent)
-    if (p.launch >= st) {
+    if (st != kResFailed && p.launch >= st) {
       const long long n = ctx->step - p.n0;
       ctx->step = p.n0;
       ctx->cur = p.cur;
       return ctx->precision == ODIS_FP64 ? step_again(ctx, ctx->d, n) : step_again(ctx, ctx->f, n);
     }
-  return fail(ctx, ODIS_E_HIP, "resident step: unknown launch taken back");
+  ctx->res_failed = 1;
+  return res_failed(ctx);
 }
 
 template <typename T>
@@ -4374,6 +4381,7 @@ static int step_t(odis_ctx *ctx, Ops<T> &o, int n_steps) {
   // dispatch-stamped start/end events (chunks with a sampled step are not
   // replayed from graphs).  The events are read by read_kernel_times when
   // the times are asked for, or before this call reuses them.
+  if (ctx->res_failed) return res_failed(ctx);
   int rc = read_kernel_times(ctx);
   if (rc) return rc;
   std::vector<ChunkEvents> sampled;

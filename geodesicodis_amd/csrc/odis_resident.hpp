@@ -400,10 +400,12 @@ __device__ __forceinline__ void res_fail(unsigned long long *ctl, unsigned *stat
   __hip_atomic_store(status, kResFailed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// Count the workgroup in and wait for the others; false when the launch was
-// taken back.  One lane of each workgroup.
+// Wait for the workgroups counted in; false when the launch was taken back,
+// or follows one that failed (the host then knows by `status`, which stays as
+// that one left it).  One lane of each workgroup.
 __device__ __forceinline__ bool res_all_here(unsigned long long *ctl, unsigned long long arrive, unsigned launch,
                                              unsigned *status) {
+  if (res_get(ctl + 1)) return false;
   const long long t0 = wall_clock64();
   unsigned long long w = res_get(ctl);
   while (!(w & kResTaken) && w < arrive) {

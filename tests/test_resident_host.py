@@ -89,3 +89,24 @@ def test_steps_of_a_launch_taken_back_are_stepped_once_each(stub, stride):
     lines = log()
     assert runs(lines) == 0 and steps(lines) == list(range(101, 151))
     """ % (stride, stride, 2 if stride else 1, stride))
+
+
+def test_a_failed_launch_leaves_no_state_to_read(stub):
+    """A workgroup that did not answer in time left the state half written:
+    the context refuses everything but its end."""
+    stub("""
+    c = ocean(2)
+    st = c.get_state()
+    S.stub_end_resident(2, 0xffffffff)
+    c.step(50)
+    c.step(50, sync=False)
+    assert refused(c.sync) == -2
+    for call in (c.sync, c.get_state, c.dissipation, lambda: c.step(1), lambda: c.step(50),
+                 lambda: c.step(1, sync=False), lambda: c.step(50, sync=False), lambda: c.velocity_en(),
+                 lambda: c.dissipation_series(0, 0, 10), lambda: c.orbit_stats([0], [10]), lambda: c.retire([0]),
+                 lambda: c.set_state(v=st["v"]), lambda: c.set_option(G.OPT_RESIDENT, 0),
+                 lambda: c.set_sh(8, np.ones(9), mode=G.SH_RECUR)):
+        assert refused(call) == -2
+    assert b"did not answer" in G.lib().odis_last_error(c._h)
+    c.close()
+    """)
