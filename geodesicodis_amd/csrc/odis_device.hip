@@ -4131,7 +4131,7 @@ static int res_patches(int N, int B, int n_cu, bool fp64, int min_W) {
 }
 
 // Patches, variant and workspace for ctx->B instances; res.off when the
-// resident step cannot run (too large for the chip).
+// resident step cannot run (too large for the chip, no memory for it).
 template <typename T>
 static int res_setup(odis_ctx *ctx) {
   ResDev &r = ctx->res;
@@ -4192,8 +4192,10 @@ static int res_setup(odis_ctx *ctx) {
   const size_t mail = size_t(r.ipl) * kResDepth * S * kResPlanes<T> * sizeof(uint4v);
   const size_t part = size_t(B) * r.chunk * W * sizeof(double);
   void *buf = nullptr;
-  if (hipMalloc(&buf, 64 + mail + part + bytes) != hipSuccess)
-    return fail(ctx, ODIS_E_NOMEM, "hipMalloc of the resident step");
+  if (hipMalloc(&buf, 64 + mail + part + bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    return ODIS_OK;  // steps are launched singly
+  }
   r.allocs.push_back(buf);
   char *const work = static_cast<char *>(buf), *const ops = work + 64 + mail + part;
   CK(hipMemset(work, 0, 64 + mail));

@@ -15,7 +15,7 @@ namespace {
 std::map<const void *, std::string> g_names;       // kernel stub -> mangled name
 std::map<void *, size_t> g_device, g_pinned;       // live allocations
 std::string g_log;
-size_t g_fail_from = 0;     // device allocations of at least this size fail (0: none)
+size_t g_fail_of = 0;       // device allocations of this size fail (0: none)
 int g_resident = 0;         // resident launches so far
 int g_end_at = 0;           // the launch that ends so (0: none), and those after it
 unsigned g_end_as = 0;      // status written: 0 its number (taken back), else the value
@@ -64,7 +64,7 @@ extern "C" {
 
 const char *stub_log() { return g_log.c_str(); }
 void stub_clear() { g_log.clear(); }
-void stub_fail_allocations_from(size_t bytes) { g_fail_from = bytes; }
+void stub_fail_allocations_of(size_t bytes) { g_fail_of = bytes; }
 // resident launch number `at` (1: the first) and later ones end with `status` (0: taken back)
 void stub_end_resident(int at, unsigned status) {
   g_end_at = at;
@@ -109,7 +109,7 @@ hipError_t hipExtLaunchKernel(const void *f, dim3 grid, dim3, void **args, size_
 }
 
 hipError_t hipMalloc(void **p, size_t n) {
-  if (g_fail_from && n >= g_fail_from) return hipErrorOutOfMemory;
+  if (g_fail_of && n == g_fail_of) return hipErrorOutOfMemory;
   *p = std::calloc(n ? n : 1, 1);
   if (!*p) return hipErrorOutOfMemory;
   g_device[*p] = n;

@@ -18,7 +18,7 @@ import ctypes, sys
 S = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
 S.stub_log.restype = ctypes.c_char_p
 S.stub_device_bytes.restype = ctypes.c_size_t
-S.stub_fail_allocations_from.argtypes = [ctypes.c_size_t]
+S.stub_fail_allocations_of.argtypes = [ctypes.c_size_t]
 S.stub_end_resident.argtypes = [ctypes.c_int, ctypes.c_uint]
 import numpy as np
 import geodesicodis_amd as G
@@ -109,4 +109,37 @@ def test_a_failed_launch_leaves_no_state_to_read(stub):
         assert refused(call) == -2
     assert b"did not answer" in G.lib().odis_last_error(c._h)
     c.close()
+    """)
+
+
+def test_no_memory_for_the_resident_step_leaves_single_launches(stub):
+    """Its workspace is optional: a context that cannot have it is created and
+    steps with a launch each; so does one that loses it in a retirement."""
+    stub("""
+    g = mesh()
+    p = G.make_params(time_step=1.0)[0]
+    def workspace(n):
+        c = G.Context(g, [p] * n)
+        c.step(20)
+        held = S.stub_device_bytes()
+        c.set_option(G.OPT_RESIDENT, 0)
+        return held - S.stub_device_bytes()
+    size = workspace(64)
+    assert size > 1 << 20
+    S.stub_fail_allocations_of(size)
+    c = G.Context(g, [p] * 64)
+    log()
+    c.step(20)
+    lines = log()
+    assert runs(lines) == 0 and steps(lines, "il") + steps(lines) == list(range(20)), lines
+    S.stub_fail_allocations_of(0)
+    d = G.Context(g, [p] * 64)
+    d.step(20)
+    assert runs(log()) == 1
+    S.stub_fail_allocations_of(workspace(63))
+    d.retire(range(63))
+    log()
+    d.step(20)
+    lines = log()
+    assert runs(lines) == 0 and steps(lines) == list(range(20, 40))
     """)
