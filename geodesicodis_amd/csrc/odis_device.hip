@@ -4097,6 +4097,7 @@ constexpr int kResCells = 641;      // cells of a patch at most
 // for 4 steps of 642 cells, 60 against 104 for 4 of 163842, FP64.
 constexpr int kResMinSteps = 4;
 constexpr size_t kResPartBytes = size_t(64) << 20;
+constexpr size_t kResLds = 160 * 1024;  // LDS of a CU
 
 static bool res_wanted(const odis_ctx *ctx) {
   return ctx->res_opt && !ctx->res.off && ctx->compact && ctx->one_kernel && ctx->patch == 64 &&
@@ -4154,9 +4155,10 @@ static int res_setup(odis_ctx *ctx) {
       const int lanes = kResVariants[v].lanes, cap = lanes * kResVariants[v].faces;
       if (h.max_cells > lanes || h.max_face > cap || h.max_bnd > lanes) continue;
       const size_t lds = res_lds_bytes<T>(lanes, h.max_cells, h.max_face, h.max_bnd, ctx->nfields);
-      if (lds > 160 * 1024) continue;
+      if (lds > kResLds) continue;
       const void *k = res_kernel<T>(ctx, v);
-      if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)) != hipSuccess) {
+      // the limit is the kernel's, shared by all contexts: always the same
+      if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, int(kResLds)) != hipSuccess) {
         (void)hipGetLastError();
         continue;
       }

@@ -143,3 +143,14 @@ def test_no_memory_for_the_resident_step_leaves_single_launches(stub):
     lines = log()
     assert runs(lines) == 0 and steps(lines) == list(range(20, 40))
     """)
+
+
+def test_lds_limit_of_a_kernel_is_the_same_for_every_context(stub):
+    """The limit belongs to the kernel, which all contexts of the process
+    share: a smaller context must not lower it under a larger one."""
+    stub("""
+    big, small = ocean(level=6, tide=G.FULL2), ocean(level=4, tide=G.NONE)
+    tiny = ocean(level=4, tide=G.FULL2, n=300)
+    limits = {tuple(x.split()[1:]) for x in log() if x.startswith("attribute ")}
+    assert limits and {v for _, v in limits} == {str(160 * 1024)}, limits
+    """)
