@@ -1668,7 +1668,7 @@ __global__ __launch_bounds__(kBlock) void k_sh_synth_rec(int L, int N, const dou
 
 // Synthesis with the rescaled recurrence: 128 cells x NW waves per
 // workgroup, each lane two cells (i, i + 64), wave g summing the orders
-// [cut[g], cut[g + 1]).  Each m sums its degrees against the degree table
+// [cut[g], cut[g + 1]) (HALVES: of eight ranges, two for each of four waves).  Each m sums its degrees against the degree table
 // (beta_l, S_l c_{l,m}, S_l c_{l,-m}) written by put_mmajor, four operations
 // per degree and cell:
 //     q_l = mu q_{l-1} + beta_l q_{l-2},  A += (S c)_{l,m} q_l,  B += (S c)_{l,-m} q_l,
@@ -1717,7 +1717,7 @@ __device__ __forceinline__ void synth_start(SynthCell<T> &c, int m, double cmm) 
   c.pmm *= T(cmm);
 }
 
-template <typename T, int NW>
+template <typename T, int NW, bool HALVES>
 __global__ __launch_bounds__(64 * NW) void k_sh_synth_chain(int L, int N, const double *__restrict__ sect,
                                                             const double *__restrict__ chain,
                                                             const double *__restrict__ trig,
@@ -1729,31 +1729,33 @@ __global__ __launch_bounds__(64 * NW) void k_sh_synth_chain(int L, int N, const 
   const int lane = threadIdx.x & 63;
   const int g = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int i0 = blockIdx.x * 128 + lane;
-  const int mlo = cut.m[g], mhi = cut.m[g + 1];
+  // orders [mlo, mhi); the rotation starts at mst, the second sum at mid
+  const int mlo = cut.m[HALVES && NW == 4 ? 2 * g : g], mhi = cut.m[HALVES && NW == 4 ? 2 * g + 2 : g + 1];
+  const int mst = HALVES && NW == 8 ? cut.m[g & ~1] : mlo, mid = HALVES && NW == 4 ? cut.m[2 * g + 1] : -1;
   SynthCell<T> u[2];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
-    const int ii = min(i0 + 64 * h, N - 1);
-    u[h].mu = T(trig[ii]);
-    u[h].s = T(trig[N + ii]);
-    u[h].cl = T(trig[2 * N + ii]);
-    u[h].sl = T(trig[3 * N + ii]);
+    const int i = min(i0 + 64 * h, N - 1);
+    u[h].mu = T(trig[i]);
+    u[h].s = T(trig[N + i]);
+    u[h].cl = T(trig[2 * N + i]);
+    u[h].sl = T(trig[3 * N + i]);
     u[h].cm = T(1);
     u[h].sm = T(0);
     u[h].pmm = T(1);
     u[h].y = T(0);
   }
+  T first[2] = {T(0), T(0)};
   if (mlo < mhi) {
     const double *e = cmaj + size_t(b) * 3 * chain_at(L, L + 1) + 3 * chain_at(L, mlo);
     if constexpr (sizeof(T) == 8) {
-      const double cmm = chain[(L + 1) * (L + 2) + mlo];
-      synth_start(u[0], mlo, cmm);
-      synth_start(u[1], mlo, cmm);
-    } else {
-      for (int q = 1; q <= mlo; ++q) {
-        synth_next_m(u[0], sect[q]);
-        synth_next_m(u[1], sect[q]);
-      }
+      const double cmm = chain[(L + 1) * (L + 2) + mst];
+      synth_start(u[0], mst, cmm);
+      synth_start(u[1], mst, cmm);
+    }
+    for (int q = sizeof(T) == 8 ? mst + 1 : 1; q <= mlo; ++q) {
+      synth_next_m(u[0], sect[q]);
+      synth_next_m(u[1], sect[q]);
     }
     T A0 = T(0), B0 = T(0), A1 = T(0), B1 = T(0);
     T p1 = T(0), p2 = u[0].pmm, r1 = T(0), r2 = u[1].pmm;
@@ -1785,6 +1787,11 @@ __global__ __launch_bounds__(64 * NW) void k_sh_synth_chain(int L, int N, const 
         synth_next_m(u[0], sect_next);
         synth_next_m(u[1], sect_next);
         ++m;
+        if (HALVES && NW == 4 && m == mid) {
+          first[0] = u[0].y;
+          first[1] = u[1].y;
+          u[0].y = u[1].y = T(0);
+        }
         left = (L - m + G) / G;
         sect_next = sect[min(m + 1, L)];
         A0 = B0 = A1 = B1 = T(0);
@@ -1794,6 +1801,10 @@ __global__ __launch_bounds__(64 * NW) void k_sh_synth_chain(int L, int N, const 
       }
     }
   }
+  if (HALVES && NW == 4) {
+    u[0].y = first[0] + u[0].y;
+    u[1].y = first[1] + u[1].y;
+  }
   part[0][threadIdx.x] = double(u[0].y);
   part[1][threadIdx.x] = double(u[1].y);
   __syncthreads();
@@ -1801,8 +1812,11 @@ __global__ __launch_bounds__(64 * NW) void k_sh_synth_chain(int L, int N, const 
   const int h = threadIdx.x >> 6, i = i0 + 64 * h;
   if (i >= N) return;
   const double *pp = part[h] + lane;
-  double sum = (pp[0] + pp[64]) + (pp[128] + pp[192]);
-  if constexpr (NW == 8) sum += (pp[256] + pp[320]) + (pp[384] + pp[448]);
+  double sum;
+  if constexpr (NW == 8)
+    sum = ((pp[0] + pp[64]) + (pp[128] + pp[192])) + ((pp[256] + pp[320]) + (pp[384] + pp[448]));
+  else
+    sum = (pp[0] + pp[64]) + (pp[128] + pp[192]);
   const T add = base ? base[b * stride + i] : T(0);
   out[b * stride + i] = add + T(sum);
 }
@@ -1811,10 +1825,13 @@ __global__ __launch_bounds__(64 * NW) void k_sh_synth_chain(int L, int N, const 
 // eight waves each, others four.  Eight against four, us: degree 32, 321
 // workgroups 11.0 / 16.6, 642 14.7 / 17.4, 963 17.5 / 18.8, 1284 23.8 / 23.1;
 // degree 16, 81 4.7 / 6.3, 642 7.0 / 7.2, 963 8.7 / 8.2, 1284 11.1 / 9.6;
-// degree 8, 642 4.8 / 4.3 (nine orders do not fill eight waves).
+// degree 8, 642 4.8 / 4.3 (nine orders do not fill eight waves).  Eight ranges
+// are cut either way and the sums are the same bit for bit: four waves run two
+// ranges each, one sum after the other, and of eight waves the odd ones rotate
+// from the start of the range before theirs, as that wave would.
 constexpr unsigned int kSynthWideBelow = 768;
 
-// Orders of the NW waves of the chain synthesis: near-equal costs, order m
+// Orders of the NW ranges of the chain synthesis: near-equal costs, order m
 // costing its groups plus kChainTurn degrees' worth for the turn to m + 1.
 constexpr int kChainTurn = 3;
 
@@ -1824,7 +1841,7 @@ static SynthCuts chain_split(int L, int NW) {
   for (int m = 0; m <= L; ++m) total += cost(m);
   SynthCuts c{};
   for (int m = 0; m <= L; ++m) {
-    // order m goes to the wave that holds its middle
+    // order m goes to the range that holds its middle
     while (g + 1 < NW && (2 * acc + cost(m)) * NW >= 2 * total * (g + 1)) c.m[++g] = m;
     acc += cost(m);
   }
@@ -3483,7 +3500,12 @@ static int sh_apply(odis_ctx *ctx, const T *x, long long stride, int nb, const d
   const bool mfma = ctx->sh_mode == ODIS_SH_MFMA;
   // cells per lane: the option, else for the pair analysis the fewest that
   // fit its grid in one round of resident workgroups, 8 for the per-degree one
-  const int cpt = ctx->sh_cpt ? ctx->sh_cpt : (by_pair ? pair_auto_cells<T>(ctx, LT, nb) : 8);
+  // (degrees without a kernel of their own take the count of one instance: it
+  // sets the order of the sums, which at these degrees is the same in any
+  // batch.  It costs batches up to 13 %: 16 instances of 40962 cells at degree
+  // 20, 174 -> 192 us per step)
+  const bool own = L == 8 || L == 16 || L == 32;
+  const int cpt = ctx->sh_cpt ? ctx->sh_cpt : (by_pair ? pair_auto_cells<T>(ctx, LT, own ? nb : 1) : 8);
   const int n_chunks = (N + 64 * cpt - 1) / (64 * cpt);
   // cmaj holds S_l c for the compiled-degree synthesis
   const double *chain = by_pair ? ctx->sh_chain : nullptr;
@@ -3551,11 +3573,12 @@ static int sh_apply(odis_ctx *ctx, const T *x, long long stride, int nb, const d
     hipEvent_t e4 = ev ? ev[4] : nullptr, e5 = ev ? ev[5] : nullptr;
     if (by_pair) {
       // FP32 contexts keep the order of their sums (see pair_degree)
-      const bool wide = sizeof(T) == 8 && L > 8 && gs2.x * nb < kSynthWideBelow;
-      const SynthCuts cut = sizeof(T) == 8 ? chain_split(L, wide ? 8 : 4) : SynthCuts{{0, mr.x, mr.y, mr.z, mr.w}};
-      hipExtLaunchKernelGGL((wide ? &k_sh_synth_chain<T, 8> : &k_sh_synth_chain<T, 4>), gs2, dim3(wide ? 512 : 256),
-                            0, ctx->stream, e4, e5, 0, L, N, ctx->sh_tabm, ctx->sh_chain, ctx->sh_trig, ctx->sh_cmaj,
-                            base, stride, out, cut);
+      const bool eight = sizeof(T) == 8 && L > 8, wide = eight && gs2.x * nb < kSynthWideBelow;
+      const SynthCuts cut = sizeof(T) == 8 ? chain_split(L, eight ? 8 : 4) : SynthCuts{{0, mr.x, mr.y, mr.z, mr.w}};
+      auto *const kernel = !eight ? &k_sh_synth_chain<T, 4, false>
+                                  : (wide ? &k_sh_synth_chain<T, 8, true> : &k_sh_synth_chain<T, 4, true>);
+      hipExtLaunchKernelGGL(kernel, gs2, dim3(wide ? 512 : 256), 0, ctx->stream, e4, e5, 0, L, N, ctx->sh_tabm,
+                            ctx->sh_chain, ctx->sh_trig, ctx->sh_cmaj, base, stride, out, cut);
     }
     else
       hipExtLaunchKernelGGL((k_sh_synth_rec<T>), gs, blk, 0, ctx->stream, e4, e5, 0, L, N, ctx->sh_tabm,

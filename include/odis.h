@@ -280,7 +280,10 @@ int odis_request_stop(odis_ctx *ctx);
  *                    32, which have compiled kernels, the fewest even count
  *                    >= 4 whose grid fits the workgroups the device holds at
  *                    once; 8 for the others), 4, 8 or 16; the coefficients depend on it by
- *                    rounding only.
+ *                    rounding only.  At degrees 8, 16 and 32 the default
+ *                    depends on the instances too; at the others, and with a
+ *                    count set, an FP64 instance steps bit for bit alike
+ *                    alone and in any batch.
  *  ODIS_OPT_INTERLEAVE a batch steps with its state held interleaved
  *                    (groups of 16 instances, instances innermost), one
  *                    workgroup per patch and 16 instances, so that the
