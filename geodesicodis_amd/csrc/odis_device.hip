@@ -2277,6 +2277,9 @@ struct ResDev {
   unsigned seq = 0, launch = 0;
   unsigned long long arrived = 0;
   int off = 0;                 // not usable on this context (or taken back once)
+  bool single = false;         // the last call's steps were launched singly
+  int few = 0;                 // calls of few steps run resident one after the other
+  long long owed = 0;          // steps of longer calls launched singly one after the other
   std::vector<void *> allocs;
   struct Pending {
     unsigned launch;
@@ -4118,7 +4121,11 @@ constexpr int kResCells = 641;      // cells of a patch at most
 // fewer steps: a launch each.  A resident call costs about 30 us beside its
 // steps (loading the ocean, the arrival, the series kernel): 40 against 42 us
 // for 4 steps of 642 cells, 60 against 104 for 4 of 163842, FP64.
+// Of a batch held interleaved a single launch does more and the line is at 2:
+// 256 x 40962 cells FP32, 0.45 ms a step, a call 0.44 and 0.17 a step.
 constexpr int kResMinSteps = 4;
+constexpr int kResFew = 3;
+static int res_min_steps(bool il) { return il ? 2 : kResMinSteps; }
 constexpr size_t kResPartBytes = size_t(64) << 20;
 constexpr size_t kResLds = 160 * 1024;  // LDS of a CU
 
@@ -4402,6 +4409,42 @@ static int res_settle(odis_ctx *ctx) {
   return res_failed(ctx);
 }
 
+// Steps after which a resident run has paid for its own cost and for the wait
+// of the next single launch (30 us), at its gain per step: 3 us at 642 cells,
+// 4 at 10242, 16 at 163842 in FP64.  Of a batch held interleaved, for the
+// conversion of its state both ways (3 steps' time each) and its own cost (one
+// step's) at a gain of 0.6 of a step.
+static int res_switch_steps(const odis_ctx *ctx, bool il) {
+  if (il) return 16;
+  const double gain = 3.0 + (ctx->precision == ODIS_FP64 ? 9e-5 : 5e-5) * ctx->N * ctx->B;
+  return std::max(kResMinSteps, int(30.0 / gain));
+}
+
+// Whether a call's steps run resident.  Changing over has a price: single
+// launches wait until the runs enqueued so far are known to have run, and of a
+// batch held interleaved the state is converted.  So singly launched steps go
+// on until calls of some steps add up to more than it, and up to kResFew calls
+// of few steps after a resident run are run resident too, which also keeps
+// them asynchronous.  us per step, asynchronous calls of 1 and 4 steps in
+// turn, changing over at each call -> so: 256 x 40962 cells FP32 881 -> 356
+// (437 launched singly), 642 cells FP64 10.7 -> 8.7.
+static bool resident_call(odis_ctx *ctx, int n_steps) {
+  ResDev &r = ctx->res;
+  const bool il = il_wanted(ctx);
+  if (!res_wanted(ctx)) return false;
+  const bool few = n_steps < res_min_steps(il);
+  if (il ? !ctx->std_fresh : r.single) {
+    r.few = 0;
+    r.owed = few ? 0 : r.owed + n_steps;
+    r.single = r.owed < res_switch_steps(ctx, il);
+  } else {
+    r.owed = 0;
+    r.few = few ? r.few + 1 : 0;
+    r.single = r.few > kResFew || (few && !il && r.pending.empty());
+  }
+  return !r.single;
+}
+
 template <typename T>
 static int step_t(odis_ctx *ctx, Ops<T> &o, int n_steps) {
   // Timing mode (ctx->timing = T > 0): the kernels of every T-th step get
@@ -4414,9 +4457,14 @@ static int step_t(odis_ctx *ctx, Ops<T> &o, int n_steps) {
   std::vector<ChunkEvents> sampled;
   size_t ev_used = 0;
   int done = 0;
-  if (res_wanted(ctx) && n_steps >= kResMinSteps && (rc = res_setup<T>(ctx))) return rc;
-  bool resident = res_wanted(ctx) && n_steps >= kResMinSteps;
-  if (!resident && ((rc = res_settle(ctx)) || (rc = enter_layout(ctx, o, il_wanted(ctx))))) return rc;
+  if (n_steps == 0) return ODIS_OK;
+  const bool il_kind = il_wanted(ctx);
+  bool resident = resident_call(ctx, n_steps);
+  if (resident) {
+    if ((rc = res_setup<T>(ctx))) return rc;
+    resident = res_wanted(ctx);
+  }
+  if (!resident && ((rc = res_settle(ctx)) || (rc = enter_layout(ctx, o, il_kind)))) return rc;
   while (done < n_steps) {
     if (ctx->stop_flag) {
       ctx->stop_flag = 0;
@@ -4431,7 +4479,7 @@ static int step_t(odis_ctx *ctx, Ops<T> &o, int n_steps) {
         const int parts = (run + ctx->res.chunk - 1) / ctx->res.chunk;
         run = (run + parts - 1) / parts;
       }
-      if (run >= kResMinSteps) {
+      if (T_s == 0 || run >= res_min_steps(il_kind) || (run > 0 && !ctx->res.pending.empty())) {
         if ((rc = enter_layout(ctx, o, false))) return rc;
         const double *table = nullptr;
         if ((rc = stage_coefficients(ctx, ctx->step, run, &table))) return rc;
@@ -4440,7 +4488,7 @@ static int step_t(odis_ctx *ctx, Ops<T> &o, int n_steps) {
         done += run;
         continue;
       }
-      if ((rc = res_settle(ctx)) || (rc = enter_layout(ctx, o, il_wanted(ctx)))) return rc;
+      if ((rc = res_settle(ctx)) || (rc = enter_layout(ctx, o, il_kind))) return rc;
       resident = res_wanted(ctx);  // not after a launch that was taken back
     }
     const bool graph_fits = ctx->use_graphs && left >= ctx->graph_steps;

@@ -154,3 +154,59 @@ def test_lds_limit_of_a_kernel_is_the_same_for_every_context(stub):
     limits = {tuple(x.split()[1:]) for x in log() if x.startswith("attribute ")}
     assert limits and {v for _, v in limits} == {str(160 * 1024)}, limits
     """)
+
+
+def test_calls_of_few_steps_after_a_run_do_not_wait(stub):
+    """Asynchronous calls stay so: the first few of fewer steps than make a
+    run are run resident behind it.  Only then does single launching, which
+    has to know that the runs took place, take over; and a call now and then
+    of some steps between single ones does not change it."""
+    stub("""
+    c = ocean()
+    c.step(200, sync=False)
+    log()
+    for n in (1, 3, 2):
+        c.step(n, sync=False)
+    lines = log()
+    assert runs(lines) == 3 and not [x for x in lines if x.startswith("wait")], lines
+    c.step(1, sync=False)
+    assert steps(log()) == [206]
+    for _ in range(3):
+        c.step(1, sync=False)
+        c.step(4, sync=False)
+    lines = log()
+    assert runs(lines) == 0 and len(steps(lines)) == 15, lines
+    c.step(100, sync=False)
+    assert runs(log()) == 1
+    assert c.get_state()["iter"] == 322
+    c.step(0)
+    """)
+
+
+def test_a_batch_is_not_converted_at_every_call(stub):
+    """Calls of one and of several steps in turn on a batch whose single steps
+    are interleaved: its state stays in the layout it has until changing over
+    pays."""
+    stub("""
+    c = ocean(16, level=7, precision=1)
+    c.step(20)
+    log()
+    for _ in range(6):
+        c.step(1)
+        c.step(4)
+    lines = log()
+    assert runs(lines) == 12 and "convert" not in lines, lines
+    for _ in range(5):
+        c.step(1)                       # now interleaved
+    lines = log()
+    assert len(steps(lines, "il")) >= 1 and lines.count("convert") == 5, lines
+    for _ in range(3):
+        c.step(1)
+        c.step(4)
+    lines = log()
+    assert len(steps(lines, "il")) == 15 and "convert" not in lines, lines
+    c.step(100)
+    lines = log()
+    assert runs(lines) == 1 and lines.count("convert") == 5, lines
+    assert c.get_state()["iter"] == 170
+    """)
