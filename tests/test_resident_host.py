@@ -210,3 +210,18 @@ def test_a_batch_is_not_converted_at_every_call(stub):
     assert runs(lines) == 1 and lines.count("convert") == 5, lines
     assert c.get_state()["iter"] == 170
     """)
+
+
+@pytest.mark.parametrize("case", ["ocean(), 1", "ocean(), 4", "ocean(16, level=7, precision=1), 8"])
+def test_steps_sampled_closely_are_staged_together(stub, case):
+    """With sampled steps closer than runs between them pay for, a call's
+    steps are one chunk, as without the resident step."""
+    stub("""
+    c, stride = %s
+    c.enable_timing(stride)
+    log()
+    c.step(64)
+    lines = log()
+    assert runs(lines) == 0 and len(steps(lines) + steps(lines, "il")) == 64
+    assert sum("k_series" in x for x in lines) == 1, lines
+    """ % case)
