@@ -41,7 +41,7 @@
 //
 // Progress: workgroups wait for each other, so all of them must be on the
 // chip.  The grid is no larger than what the chip holds, resident launches of
-// one process follow one another on the device, and the first thing a launch does is to count
+// one process that would not fit together follow one another, and the first thing a launch does is to count
 // its workgroups in: until the count is complete nothing has been written,
 // and if it is not complete in time (another process holds the CUs) one
 // workgroup takes the launch back -- one atomic word decides between

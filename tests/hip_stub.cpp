@@ -18,6 +18,7 @@ std::string g_log;
 size_t g_fail_of = 0;       // device allocations of this size fail (0: none)
 int g_resident = 0;         // resident launches so far
 int g_end_at = 0;           // the launch that ends so (0: none), and those after it
+int g_per_cu = 1;           // workgroups a compute unit holds
 unsigned g_end_as = 0;      // status written: 0 its number (taken back), else the value
 unsigned g_status = 0;      // as the device holds it: written once
 dim3 g_grid, g_block;
@@ -70,6 +71,7 @@ void stub_end_resident(int at, unsigned status) {
   g_end_at = at;
   g_end_as = status;
 }
+void stub_workgroups_per_cu(int n) { g_per_cu = n; }
 size_t stub_device_bytes() {
   size_t n = 0;
   for (const auto &b : g_device) n += b.second;
@@ -162,7 +164,7 @@ hipError_t hipFuncSetAttribute(const void *f, hipFuncAttribute, int v) {
   return hipSuccess;
 }
 hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int *n, const void *, int, size_t) {
-  *n = 1;
+  *n = g_per_cu;
   return hipSuccess;
 }
 

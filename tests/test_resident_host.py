@@ -225,3 +225,45 @@ def test_steps_sampled_closely_are_staged_together(stub, case):
     assert runs(lines) == 0 and len(steps(lines) + steps(lines, "il")) == 64
     assert sum("k_series" in x for x in lines) == 1, lines
     """ % case)
+
+
+def test_launches_of_several_contexts_are_ordered_only_where_they_must_be(stub):
+    """Launches whose workgroups fit the chip together are not ordered; one
+    that does not fit waits for each launch of the group before it."""
+    stub("""
+    g, g4 = mesh(6), mesh(4)
+    p = G.make_params(time_step=1.0)[0]
+
+    def context(patches):
+        c = G.Context(g if patches > 16 else g4, [p])
+        c.set_option(G.OPT_RESIDENT, patches)
+        return c
+
+    def waits(c):
+        log()
+        c.step(8, sync=False)
+        return sum(x == "after another launch" for x in log())
+    small = [ocean() for _ in range(8)]          # 16 workgroups each
+    assert [waits(c) for c in small + small] == [0] * 16
+    for c in small:
+        c.close()
+    a, x, z, v = context(200), context(100), context(150), context(2)
+    assert waits(a) == 0
+    assert waits(x) == 1                         # after a
+    assert waits(z) == 1                         # beside x, after a
+    assert [waits(c) for c in (x, z, x)] == [0] * 3
+    assert waits(a) == 2                         # after x and z
+    assert waits(v) == 2                         # beside a, after x and z
+    assert waits(x) == 2                         # after a and v
+    assert waits(z) == 2                         # beside x
+    assert waits(v) == 1                         # beside x and z, after a (its own is before it anyway)
+    w = context(3)
+    assert waits(w) == 2                         # after a and v's launch in a's group
+    # the newest group's contexts end: what follows still waits for the group before
+    assert waits(a) == 4
+    a.close()
+    S.stub_workgroups_per_cu(2)
+    y = ocean(40)                                # more workgroups than compute units
+    assert waits(y) == 4
+    assert waits(x) == 1
+    """)
