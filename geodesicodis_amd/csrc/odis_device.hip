@@ -3086,7 +3086,10 @@ static int create_impl(const odis_mesh_desc *m, const odis_params *params, int n
     if (he == hipSuccess) he = hipDeviceSynchronize();
     if (he != hipSuccess) rc = fail(ctx, ODIS_E_HIP, hipGetErrorString(he));
   }
-  if (!rc && res_wanted(ctx)) rc = precision == ODIS_FP64 ? res_setup<double>(ctx) : res_setup<float>(ctx);
+  // the resident step, unless the surface is one that a basis will be set for
+  // (1 ms at 10242 cells, 5 at 163842; at the first run if none is)
+  if (!rc && res_wanted(ctx) && params[0].surface == ODIS_FREE)
+    rc = precision == ODIS_FP64 ? res_setup<double>(ctx) : res_setup<float>(ctx);
   *building = nullptr;
   if (rc) {
     const std::string msg = ctx->err;
@@ -5264,6 +5267,11 @@ static int sh_set_basis_impl(odis_ctx *ctx, int l_max, const double *beta, int m
   if (settled) return settled;
   CK(hipStreamSynchronize(ctx->stream));
   drop_graphs(ctx);
+  if (mode != ODIS_SH_OFF) {  // no resident step with a basis
+    const int off = ctx->res.off;
+    res_free(ctx);
+    ctx->res.off = off;
+  }
   for (void *p : ctx->sh_allocs) (void)hipFree(p);
   ctx->sh_allocs.clear();
   ctx->sh_mode = ODIS_SH_OFF;

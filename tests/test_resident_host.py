@@ -267,3 +267,29 @@ def test_launches_of_several_contexts_are_ordered_only_where_they_must_be(stub):
     assert waits(y) == 4
     assert waits(x) == 1
     """)
+
+
+def test_a_shell_holds_no_resident_step(stub):
+    """Contexts coupled through spherical harmonics never run it: those that
+    will be by their surface do not set it up when created, others give it back
+    when a basis is set; without a basis they run it."""
+    stub("""
+    def grown(call):
+        before = S.stub_device_bytes()
+        out = call()
+        return out, S.stub_device_bytes() - before
+    free, b0 = grown(lambda: ocean(8))
+    lid, b1 = grown(lambda: ocean(8, surface=G.LID_MEMBR, shell_thickness=20e3))
+    load, b2 = grown(lambda: ocean(8, surface=G.FREE_LOADING))
+    workspace = b0 - b1
+    assert workspace > 1 << 19 and b1 == b2
+    # (the stub computes no basis: the call ends with an error once it has the Gram matrix)
+    _, f = grown(lambda: refused(lambda: free.set_sh(8, np.ones(9), mode=G.SH_RECUR)))
+    _, l = grown(lambda: refused(lambda: lid.set_sh(8, np.ones(9), mode=G.SH_RECUR)))
+    assert l - f == workspace
+    for c in (free, lid, load):
+        c.set_sh(8, np.ones(9), mode=G.SH_OFF)
+        log()
+        c.step(20)
+        assert runs(log()) == 1
+    """)
