@@ -49,6 +49,7 @@ SH_OFF, SH_FP64, SH_SPLIT_BF16, SH_RECUR, SH_MFMA = 0, 1, 2, 3, 4
 OPT_GRAPHS, OPT_COMPACT, OPT_ONE_KERNEL, OPT_PATCH_CELLS, OPT_STEP_BLOCKS, OPT_STEP_LANES, OPT_SH_CELLS = \
     1, 2, 3, 4, 5, 6, 7
 OPT_INTERLEAVE, OPT_INTERLEAVE_ACTIVE, OPT_IL_UNROLL, OPT_IL_ORDER, OPT_IL_RECORDS, OPT_RESIDENT = 8, 9, 10, 11, 12, 13
+OPT_RESIDENT_ACTIVE, OPT_RESIDENT_MISS = 14, 15
 
 
 class OdisError(RuntimeError):

@@ -2333,6 +2333,7 @@ struct odis_ctx {
   // resident launches (many steps per launch, odis_resident.hpp)
   int res_opt = 1;             // ODIS_OPT_RESIDENT: 0 off, 1 automatic, > 1 that many patches per instance
   ResDev res;
+  int res_miss = 0;            // ODIS_OPT_RESIDENT_MISS: launches up to the one that waits in vain
   int res_failed = 0;          // a resident launch ended partway: the state is lost
   std::string one_kernel_why;
   std::vector<int> gi_host, cyc_host;  // device-order face cells and cell cycles, to rebuild patches
@@ -4314,6 +4315,7 @@ static int launch_resident(odis_ctx *ctx, Ops<T> &o, const double *table, int co
   const unsigned grid = unsigned(r.ipl) * unsigned(r.W);
   r.arrived += grid;
   a.arrive = r.arrived;
+  if (ctx->res_miss > 0 && --ctx->res_miss == 0) a.arrive++;
   a.g_coef = o.g_coef;
   a.fcor = o.fcor;
   a.farea = o.farea;
@@ -4874,11 +4876,16 @@ static int set_option_impl(odis_ctx *ctx, int option, int value) {
   if (settled) return settled;
   if (option == ODIS_OPT_RESIDENT) {
     if (value < 0) return fail(ctx, ODIS_E_INVALID, "resident steps: 0 (off), 1 (automatic) or the patches per instance");
-    if (value != ctx->res_opt) {
+    if (value != ctx->res_opt || ctx->res.off) {  // set up again, also after a launch that was taken back
       CK(hipStreamSynchronize(ctx->stream));
       res_free(ctx);
       ctx->res_opt = value;
     }
+    return ODIS_OK;
+  }
+  if (option == ODIS_OPT_RESIDENT_MISS) {
+    if (value < 0) return fail(ctx, ODIS_E_INVALID, "number of the launch, or 0");
+    ctx->res_miss = value;
     return ODIS_OK;
   }
   if (option == ODIS_OPT_GRAPHS) {
@@ -4998,6 +5005,8 @@ extern "C" int odis_get_option(odis_ctx *ctx, int option, int *value) {
   else if (option == ODIS_OPT_IL_ORDER) *value = ctx->il_order;
   else if (option == ODIS_OPT_IL_RECORDS) *value = ctx->il_rec;
   else if (option == ODIS_OPT_RESIDENT) *value = ctx->res_opt;
+  else if (option == ODIS_OPT_RESIDENT_ACTIVE) *value = res_wanted(ctx) ? ctx->res.W : 0;
+  else if (option == ODIS_OPT_RESIDENT_MISS) *value = ctx->res_miss;
   else return fail(ctx, ODIS_E_INVALID, "unknown option");
   return ODIS_OK;
 }

@@ -319,10 +319,21 @@ int odis_request_stop(odis_ctx *ctx);
  *                    LDS of one workgroup per patch: 1 (default) when the
  *                    ocean fits the chip, no SH basis is set, the launch
  *                    options above are at their defaults (interleaving 0 or
- *                    2) and an odis_step call has enough steps; 0 off; a
+ *                    2) and the steps are enough to pay for it; 0 off; a
  *                    larger value: that many patches per instance.  Steps
  *                    sampled for timing are launched by themselves.  Same
- *                    state bit for bit; dissipation sums differ by rounding. */
+ *                    state bit for bit; dissipation sums differ by rounding.
+ *                    When another process holds a part of the chip, a launch
+ *                    is taken back, its steps and the later ones are launched
+ *                    singly, and so are all others until the option is set
+ *                    again (to the same value or another).
+ *  ODIS_OPT_RESIDENT_ACTIVE (read only) the patches per instance of the
+ *                    resident step that is set up, 0 when steps are launched
+ *                    singly.  Set up at creation, of oceans whose surface
+ *                    takes an SH basis at the first run without one.
+ *  ODIS_OPT_RESIDENT_MISS (for tests) n > 0: the n-th resident launch from
+ *                    here waits for one workgroup more than it has, and so
+ *                    is taken back after 0.2 s. */
 #define ODIS_OPT_GRAPHS     1
 #define ODIS_OPT_COMPACT    2
 #define ODIS_OPT_ONE_KERNEL 3
@@ -336,6 +347,8 @@ int odis_request_stop(odis_ctx *ctx);
 #define ODIS_OPT_IL_ORDER 11
 #define ODIS_OPT_IL_RECORDS 12
 #define ODIS_OPT_RESIDENT 13
+#define ODIS_OPT_RESIDENT_ACTIVE 14
+#define ODIS_OPT_RESIDENT_MISS 15
 int odis_set_option(odis_ctx *ctx, int option, int value);
 int odis_get_option(odis_ctx *ctx, int option, int *value);
 /* Timing for benchmarks: with stride T > 0, the kernels of every step n of

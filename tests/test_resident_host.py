@@ -14,7 +14,7 @@ from conftest import ROOT
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 PRELUDE = """
-import ctypes, sys
+import ctypes, functools, sys
 S = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
 S.stub_log.restype = ctypes.c_char_p
 S.stub_device_bytes.restype = ctypes.c_size_t
@@ -34,6 +34,7 @@ def steps(lines, kind="step"):
 def runs(lines):
     return sum(x.startswith("resident ") for x in lines)
 
+@functools.lru_cache(None)
 def mesh(level=4):
     return G.Mesh(G.Grid.generate(level, 64), 252.1e3)
 
@@ -292,4 +293,41 @@ def test_a_shell_holds_no_resident_step(stub):
         log()
         c.step(20)
         assert runs(log()) == 1
+    """)
+
+
+def test_the_resident_step_in_use_can_be_read_and_tried_again(stub):
+    stub("""
+    c = ocean()
+    assert c.option(G.OPT_RESIDENT_ACTIVE) == 16                     # 642 / 40 cells
+    c.set_option(G.OPT_GRAPHS, 1)
+    assert c.option(G.OPT_RESIDENT_ACTIVE) == 0
+    c.set_option(G.OPT_GRAPHS, 0)
+    S.stub_end_resident(1, 0)
+    c.step(20)
+    assert c.option(G.OPT_RESIDENT_ACTIVE) == 0 and c.option(G.OPT_RESIDENT) == 1
+    S.stub_end_resident(0, 0)
+    c.set_option(G.OPT_RESIDENT, 1)
+    log()
+    c.step(20)
+    assert runs(log()) == 1 and c.option(G.OPT_RESIDENT_ACTIVE) == 16
+    assert refused(lambda: c.set_option(G.OPT_RESIDENT_ACTIVE, 1)) == -1
+    assert ocean(3, level=2).option(G.OPT_RESIDENT_ACTIVE) >= 1     # 42 cells: one patch
+    # 163842 cells in FP64 with 7 tide fields are more than the chip's LDS holds
+    assert ocean(level=8, tide=G.FULL2).option(G.OPT_RESIDENT_ACTIVE) == 0
+    """)
+
+
+def test_a_stop_does_not_end_steps_already_taken(stub):
+    """Steps accepted before a stop was requested are stepped again when their
+    launch was taken back; the stop ends the next call."""
+    stub("""
+    c = ocean()
+    S.stub_end_resident(1, 0)
+    c.step(50, sync=False)
+    G.lib().odis_request_stop(c._h)
+    assert c.get_state()["iter"] == 50
+    assert refused(lambda: c.step(10)) == -7
+    c.step(10)
+    assert c.get_state()["iter"] == 60
     """)
