@@ -3,31 +3,35 @@
 The step kernels have launch shapes that only the device can rank: the
 one-kernel step or the face + cell pair, cells per patch, lanes per cell,
 the interleaved batch layout with the faces / (cell, instance) pairs each
-lane keeps in flight, its workgroup order and its operand records, and
-HIP-graph replay.  Every candidate gives the same
+lane keeps in flight, its workgroup order and its operand records, HIP-graph
+replay, and the resident step, which runs where those are at their defaults.
+Every candidate gives the same
 state bit for bit (dissipation sums differ by rounding), so tuning never
 changes results.
 
 tune() times each candidate on a scratch context of the same mesh, batch,
 precision and SH coupling (the caller's context is not stepped), keeps the
 fastest, and caches the choice per (cells, instances, precision, SH mode,
-degree, device) in memory and in a JSON file (ODIS_TUNE_CACHE, else
+degree, build of the library, device) in memory and in a JSON file (ODIS_TUNE_CACHE, else
 ~/.cache/geodesicodis_amd/tune.json).  A candidate replaces the default only
 when it is at least `margin` faster.
 """
+import functools
+import hashlib
 import itertools
 import json
 import os
 import time
 
-from . import (FP64, OPT_GRAPHS, OPT_IL_ORDER, OPT_IL_RECORDS, OPT_IL_UNROLL, OPT_INTERLEAVE,
-               OPT_INTERLEAVE_ACTIVE, OPT_ONE_KERNEL, OPT_PATCH_CELLS, OPT_STEP_LANES, SH_OFF, Context, OdisError)
+from . import (FP64, LIB_PATH, OPT_GRAPHS, OPT_IL_ORDER, OPT_IL_RECORDS, OPT_IL_UNROLL, OPT_INTERLEAVE,
+               OPT_INTERLEAVE_ACTIVE, OPT_ONE_KERNEL, OPT_PATCH_CELLS, OPT_RESIDENT, OPT_STEP_LANES, SH_OFF, Context,
+               OdisError)
 
 TUNED = (OPT_ONE_KERNEL, OPT_PATCH_CELLS, OPT_STEP_LANES, OPT_INTERLEAVE, OPT_IL_UNROLL, OPT_IL_ORDER, OPT_IL_RECORDS,
-         OPT_GRAPHS)
+         OPT_GRAPHS, OPT_RESIDENT)
 NAMES = {OPT_ONE_KERNEL: "one_kernel", OPT_PATCH_CELLS: "patch_cells", OPT_STEP_LANES: "step_lanes",
          OPT_INTERLEAVE: "interleave", OPT_IL_UNROLL: "il_unroll", OPT_IL_ORDER: "il_order",
-         OPT_IL_RECORDS: "il_records", OPT_GRAPHS: "graphs"}
+         OPT_IL_RECORDS: "il_records", OPT_GRAPHS: "graphs", OPT_RESIDENT: "resident"}
 
 _MEMO = {}
 
@@ -57,6 +61,13 @@ def _store_cache(key, entry):
         os.replace(tmp, path)
     except OSError:
         pass  # a read-only home: the in-memory cache still holds it
+
+
+@functools.lru_cache(maxsize=None)
+def _build(path):
+    """The library's build: times of one say nothing about another."""
+    with open(path, "rb") as fh:
+        return hashlib.sha1(fh.read()).hexdigest()[:12]
 
 
 def _device_name():
@@ -103,9 +114,7 @@ def apply(ctx, options):
     """Set option values (a dict option -> value) on a context; options the
     context refuses are left as they are.  Returns the options set."""
     done = {}
-    order = (OPT_ONE_KERNEL, OPT_PATCH_CELLS, OPT_STEP_LANES, OPT_INTERLEAVE, OPT_IL_UNROLL, OPT_IL_ORDER,
-             OPT_IL_RECORDS, OPT_GRAPHS)
-    for o in order:
+    for o in TUNED:
         if o in options:
             try:
                 ctx.set_option(o, int(options[o]))
@@ -133,8 +142,8 @@ def tune(mesh, params, precision=FP64, sh=None, steps=100, warmup=20, repeats=3,
     option_ids()), "ms_per_step" tuned and "default_ms_per_step", "speedup",
     "candidates" timed, "cached"."""
     params = list(params)
-    key = "%d/%d/%d/%s/%d/%s%s" % (mesh.N, len(params), precision, sh[2] if sh else SH_OFF,
-                                   sh[0] if sh else 0, _device_name(), "" if graphs else "/no-graphs")
+    key = "%d/%d/%d/%s/%d/%s/%s%s" % (mesh.N, len(params), precision, sh[2] if sh else SH_OFF, sh[0] if sh else 0,
+                                      _build(LIB_PATH), _device_name(), "" if graphs else "/no-graphs")
     if use_cache:
         if key in _MEMO:
             return dict(_MEMO[key], cached=True)

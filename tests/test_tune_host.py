@@ -167,3 +167,43 @@ def test_tune_cache_survives_a_corrupt_file(fake_tuner, monkeypatch):
     r = T.tune(_Mesh, [object()])
     assert not r["cached"]
     assert len(json.loads(fake_tuner.read_text())) == 1
+
+
+def test_a_choice_of_another_build_is_not_used(fake_tuner, monkeypatch, tmp_path):
+    """A cached choice belongs to the build it was timed on: the kernels of
+    another rank otherwise, and a choice made before a step existed would
+    switch that step off."""
+    libs = [tmp_path / "a.so", tmp_path / "b.so"]
+    for k, so in enumerate(libs):
+        so.write_bytes(b"build %d" % k)
+    monkeypatch.setattr(T, "_time", _timer([({G.OPT_ONE_KERNEL: 0, G.OPT_GRAPHS: 0}, 0.5)]))
+    monkeypatch.setattr(T, "LIB_PATH", str(libs[0]))
+    assert not T.tune(_Mesh, [object()] * 2)["cached"]
+    assert T.tune(_Mesh, [object()] * 2)["cached"]
+    monkeypatch.setattr(T, "LIB_PATH", str(libs[1]))
+    assert not T.tune(_Mesh, [object()] * 2)["cached"]
+    monkeypatch.setattr(T, "_MEMO", {})
+    monkeypatch.setattr(T, "LIB_PATH", str(libs[0]))
+    assert T.tune(_Mesh, [object()] * 2)["cached"]           # from the file
+    assert len(json.loads(fake_tuner.read_text())) == 2
+
+
+def test_a_choice_sets_the_resident_step(fake_tuner, monkeypatch):
+    """The resident step is part of a choice, so that applying it does not
+    leave a context's own setting in the way of what was timed."""
+    monkeypatch.setattr(FakeContext, "__init__", _with_resident(FakeContext.__init__))
+    monkeypatch.setattr(T, "_time", _timer([({G.OPT_RESIDENT: 1, G.OPT_PATCH_CELLS: 64, G.OPT_STEP_LANES: 4,
+                                             G.OPT_GRAPHS: 0}, 0.3)]))
+    r = T.tune(_Mesh, [object()], use_cache=False)
+    assert r["options"]["resident"] == 1 and r["speedup"] == 1.0
+    ctx = FakeContext(B=1)
+    ctx.opts[G.OPT_RESIDENT] = 0
+    T.apply(ctx, T.option_ids(r["options"]))
+    assert ctx.option(G.OPT_RESIDENT) == 1
+
+
+def _with_resident(init):
+    def made(self, *a, **kw):
+        init(self, *a, **kw)
+        self.opts[G.OPT_RESIDENT] = 1
+    return made
