@@ -38,7 +38,8 @@ sweep` and `--workload uneven` run one batched extra alone (for profiling).
 
 Prints one JSON line: cell-steps/s of the whole job; the roofline of the
 dominant kernel (HIP events stamped on the kernel dispatches of every 64th
-step of a long run, inside the timed region); and a CPU baseline (the FP64 C oracle with
+step of a long run, inside the timed region; of a free-surface ocean, whose
+steps run many to a launch, in a run of single launches); and a CPU baseline (the FP64 C oracle with
 OpenMP, with the same projection as dense products, on a bounded sample of
 the same workload).
 """
@@ -176,6 +177,23 @@ def timed_run(ctx, steps, warmup, stride):
     tm = ctx.timing()
     ctx.enable_timing(0)
     return elapsed, tm
+
+
+def timed_kernels(G, make_ctx, args):
+    """(context, seconds, kernel times, patches) of the run's steps on a
+    context of make_ctx's.  A resident run is one kernel for many steps: it is
+    timed with no step sampled, the kernels of a step launched by itself on
+    another context; its patches per instance tell (0: steps launched singly)."""
+    ctx = make_ctx()
+    patches = ctx.option(G.OPT_RESIDENT_ACTIVE)
+    if not patches:
+        return (ctx,) + timed_run(ctx, args.steps, args.warmup, args.timing_stride) + (0,)
+    elapsed, _ = timed_run(ctx, args.steps, args.warmup, 0)
+    other = make_ctx()
+    other.set_option(G.OPT_RESIDENT, 0)
+    _, tm = timed_run(other, args.steps, args.warmup, args.timing_stride)
+    other.close()
+    return ctx, elapsed, tm, patches
 
 
 def shell_setup(G):
@@ -748,8 +766,7 @@ def main():
 
     prec = G.FP64 if args.precision == "fp64" else G.FP32
     p_bytes = 8 if prec == G.FP64 else 4
-    ctx = make_ctx(prec)
-    elapsed, tm = timed_run(ctx, args.steps, args.warmup, args.timing_stride)
+    ctx, elapsed, tm, patches = timed_kernels(G, lambda: make_ctx(prec), args)
     ms_per_step = 1e3 * elapsed / args.steps
     value = mesh.N * args.steps / elapsed
     diss = ctx.dissipation()
@@ -833,7 +850,9 @@ def main():
             "sh_basis": (("on the fly (Legendre recurrence, %s)" % ("fp64" if prec == G.FP64 else "fp32")) if recur
                          else ("stored fp64" if prec == G.FP64 else "stored split-bf16")) if shell else None,
             "trisk": "cell-local (kite fractions)" if ctx.option(G.OPT_COMPACT) else "tabulated",
-            "launch": ("SH analysis, partial sums, coefficients, synthesis + " if shell else "") +
+            "launch": "resident: many steps per launch, %d patches (kernels and roofline: a step launched by itself)"
+                      % patches if patches else
+                      ("SH analysis, partial sums, coefficients, synthesis + " if shell else "") +
                       (("one stencil kernel per step (patches of <= %d cells, %d lanes per cell, %d workgroups)"
                         % (ctx.option(G.OPT_PATCH_CELLS), ctx.option(G.OPT_STEP_LANES),
                            ctx.option(G.OPT_STEP_BLOCKS))) if one else "face + cell kernel per step"),
@@ -846,7 +865,7 @@ def main():
             "step_events_ms": tm["step_ms"],
             "alg_bytes": alg,
             "alg_bytes_per_step": step_bytes,
-            "hbm_gbs_per_step": step_bytes / (ms_per_step * 1e-3) / 1e9,
+            "hbm_gbs_per_step": None if patches else step_bytes / (ms_per_step * 1e-3) / 1e9,
             "dissipation_W_m2": float(diss[0]),
         },
         "roofline": {
@@ -911,16 +930,20 @@ def main():
             pf, _ = G.make_params(time_step=6.5)
             fmesh = G.Mesh(grid, pf.radius)
             for name, fprec in (("free_surface_fp64", G.FP64), ("free_surface_fp32", G.FP32)):
-                c2 = G.Context(fmesh, pf, precision=fprec)
-                apply_launch_options(G, c2, args)
-                el2, tm2 = timed_run(c2, args.steps, args.warmup, args.timing_stride)
+                def free_ctx(fprec=fprec):
+                    c = G.Context(fmesh, pf, precision=fprec)
+                    apply_launch_options(G, c, args)
+                    return c
+                c2, el2, tm2, patches2 = timed_kernels(G, free_ctx, args)
                 one2 = c2.option(G.OPT_ONE_KERNEL) == 1
                 tn2 = ("double" if fprec == G.FP64 else "float") + ",compact"
                 kn, kb, km, _ = stencil_roofline(G, c2, fmesh, tm2, 8 if fprec == G.FP64 else 4, one2)
                 out["config"][name] = {
                     "value": fmesh.N * args.steps / el2, "ms_per_step": 1e3 * el2 / args.steps,
-                    "kernel": "%s<%s>" % (kn, tn2), "kernel_ms": km, "alg_bytes": kb,
-                    "hbm_frac": (kb / (km * 1e-3) / 1e9 / HBM_PEAK_GBS) if km > 0 else None}
+                    "resident_patches": patches2,
+                    "single_launch": {
+                        "kernel": "%s<%s>" % (kn, tn2), "kernel_ms": km, "alg_bytes": kb,
+                        "hbm_frac": (kb / (km * 1e-3) / 1e9 / HBM_PEAK_GBS) if km > 0 else None}}
                 c2.close()
 
     if not args.no_extra and not args.no_sweep:

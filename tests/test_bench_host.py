@@ -100,3 +100,55 @@ def test_more_than_one_gpu_is_refused():
     r = subprocess.run([sys.executable, os.path.join(root, "bench.py"), "--gpus", "2"], capture_output=True,
                        text=True, timeout=120)
     assert r.returncode == 2 and "exactly one GPU" in r.stderr and r.stdout == ""
+
+
+class _Ctx:
+    """A context's side of a timed run: the options, the sampling stride of
+    each odis_step call."""
+    def __init__(self, G, patches):
+        self.G, self.opts, self.strides, self.stride = G, {G.OPT_RESIDENT: 1}, [], 0
+        self.patches, self.closed = patches, False
+
+    def option(self, o):
+        return self.patches * (self.opts[self.G.OPT_RESIDENT] > 0) if o == self.G.OPT_RESIDENT_ACTIVE else self.opts[o]
+
+    def set_option(self, o, v):
+        self.opts[o] = v
+
+    def enable_timing(self, stride):
+        self.stride = stride
+
+    def step(self, n, sync=True):
+        self.strides.append((n, self.stride))
+
+    def timing(self):
+        return {"step_ms": 0.02 if self.stride else 0.0}
+
+    def sync(self):
+        pass
+
+    def close(self):
+        self.closed = True
+
+
+def test_resident_steps_are_timed_unsampled_and_kernels_apart():
+    """The timed steps of a context that runs resident are not cut by sampled
+    ones, and the kernel times are those of another that launches singly; a
+    context that launches singly gives both."""
+    import types
+
+    import geodesicodis_amd as G
+    args = types.SimpleNamespace(steps=100, warmup=5, timing_stride=16)
+    for patches in (0, 256):
+        made = []
+
+        def make():
+            made.append(_Ctx(G, patches))
+            return made[-1]
+        ctx, _, tm, got = bench.timed_kernels(G, make, args)
+        assert ctx is made[0] and got == patches and tm["step_ms"] == 0.02 and not ctx.closed
+        if patches:
+            assert ctx.strides == [(5, 0), (100, 0)] and ctx.opts[G.OPT_RESIDENT] == 1
+            assert made[1].strides == [(5, 16), (100, 16)] and made[1].opts[G.OPT_RESIDENT] == 0 and made[1].closed
+        else:
+            assert ctx.strides == [(5, 16), (100, 16)] and len(made) == 1
