@@ -54,6 +54,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <future>
 #include <string>
 #include <system_error>
@@ -133,6 +134,8 @@ inline void bisect_cells(ResPoint *pt, int lo, int hi, int j, int W, std::vector
 inline std::string build_resident(int N, int E, const std::vector<float> &xyz, const std::vector<int> &gi,
                                   const std::vector<int> &cyc, int W, ResHost &h) {
   h.W = W;
+  for (float x : xyz)
+    if (!std::isfinite(x)) return "a cell without a place";
   h.cptr.assign(W + 1, 0);
   std::vector<int> patch(N);
   std::vector<ResPoint> pt(N);

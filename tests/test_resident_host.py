@@ -331,3 +331,23 @@ def test_a_stop_does_not_end_steps_already_taken(stub):
     c.step(10)
     assert c.get_state()["iter"] == 60
     """)
+
+
+def test_cells_without_a_place_step_singly(stub):
+    """Cell coordinates only order the cells and their patches; a descriptor
+    whose coordinates are no numbers is still a mesh, but has no patches (NaN
+    has no place in the order that cuts them)."""
+    stub("""
+    g = mesh()
+    d = g.describe()
+    lat = np.ctypeslib.as_array(ctypes.cast(d.cell_lat, ctypes.POINTER(ctypes.c_double)), (g.N,)).copy()
+    lat[::3] = np.nan
+    d.cell_lat = type(d.cell_lat)(lat.ctypes.data) if not hasattr(d.cell_lat, "contents") else \\
+        lat.ctypes.data_as(type(d.cell_lat))
+    g.describe = lambda: d
+    c = G.Context(g, G.make_params(time_step=1.0)[0])
+    assert c.option(G.OPT_RESIDENT_ACTIVE) == 0
+    log()
+    c.step(20)
+    assert steps(log()) == list(range(20))
+    """)
