@@ -1668,9 +1668,9 @@ __global__ __launch_bounds__(kBlock) void k_sh_synth_rec(int L, int N, const dou
 
 // Synthesis with the rescaled recurrence: 128 cells x NW waves per
 // workgroup, each lane two cells (i, i + 64), wave g summing the orders
-// [cut[g], cut[g + 1]) (HALVES: of eight ranges, two for each of four waves).  Each m sums its degrees against the degree table
-// (beta_l, S_l c_{l,m}, S_l c_{l,-m}) written by put_mmajor, four operations
-// per degree and cell:
+// [cut[g], cut[g + 1]) (HALVES: of eight ranges, two for each of four waves).
+// Each m sums its degrees against the degree table (beta_l, S_l c_{l,m}, S_l
+// c_{l,-m}) written by put_mmajor, four operations per degree and cell:
 //     q_l = mu q_{l-1} + beta_l q_{l-2},  A += (S c)_{l,m} q_l,  B += (S c)_{l,-m} q_l,
 // from q_{m-1} = 0, q_{m-2} = P_mm (beta_m = 1, beta_{m+1} = 0), and
 // y = sum_m A_m cos(m lon) + B_m sin(m lon); the waves' sums are added
@@ -1723,15 +1723,15 @@ __global__ __launch_bounds__(64 * NW) void k_sh_synth_chain(int L, int N, const 
                                                             const double *__restrict__ trig,
                                                             const double *__restrict__ cmaj, const T *base,
                                                             long long stride, T *out, SynthCuts cut) {
-  constexpr int G = kChainGroup;
+  constexpr int G = kChainGroup, kHalves = HALVES && NW == 4 ? 2 : 1;
   __shared__ double part[2][64 * NW];
   const int b = blockIdx.y;
   const int lane = threadIdx.x & 63;
   const int g = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int i0 = blockIdx.x * 128 + lane;
   // orders [mlo, mhi); the rotation starts at mst, the second sum at mid
-  const int mlo = cut.m[HALVES && NW == 4 ? 2 * g : g], mhi = cut.m[HALVES && NW == 4 ? 2 * g + 2 : g + 1];
-  const int mst = HALVES && NW == 8 ? cut.m[g & ~1] : mlo, mid = HALVES && NW == 4 ? cut.m[2 * g + 1] : -1;
+  const int mlo = cut.m[kHalves * g], mhi = cut.m[kHalves * (g + 1)], mid = cut.m[kHalves * g + 1];
+  const int mst = HALVES && NW == 8 ? cut.m[g & ~1] : mlo;
   SynthCell<T> u[2];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
@@ -1761,49 +1761,51 @@ __global__ __launch_bounds__(64 * NW) void k_sh_synth_chain(int L, int N, const 
     T p1 = T(0), p2 = u[0].pmm, r1 = T(0), r2 = u[1].pmm;
     int m = mlo, left = (L - m + G) / G;
     double sect_next = sect[min(m + 1, L)];
-    const int total = chain_groups(L + 1 - mlo) - chain_groups(L + 1 - mhi);
 #pragma unroll 1
-    for (int q = 0; q < total; ++q, e += 3 * G) {
-      double cur[3 * G];
+    for (int half = 0; half < kHalves; ++half) {
+      const int hi = half + 1 < kHalves ? mid : mhi;
+      const int total = chain_groups(L + 1 - m) - chain_groups(L + 1 - hi);
+#pragma unroll 1
+      for (int q = 0; q < total; ++q, e += 3 * G) {
+        double cur[3 * G];
 #pragma unroll
-      for (int k = 0; k < 3 * G; ++k) cur[k] = e[k];
+        for (int k = 0; k < 3 * G; ++k) cur[k] = e[k];
 #pragma unroll
-      for (int k = 0; k < G; ++k) {
-        const T be = T(cur[3 * k]), cc = T(cur[3 * k + 1]), ss = T(cur[3 * k + 2]);
-        const T p = fma(u[0].mu, p1, be * p2);
-        const T r = fma(u[1].mu, r1, be * r2);
-        p2 = p1;
-        p1 = p;
-        r2 = r1;
-        r1 = r;
-        A0 = fma(cc, p, A0);
-        B0 = fma(ss, p, B0);
-        A1 = fma(cc, r, A1);
-        B1 = fma(ss, r, B1);
-      }
-      if (--left == 0) {
-        u[0].y = fma(B0, u[0].sm, fma(A0, u[0].cm, u[0].y));
-        u[1].y = fma(B1, u[1].sm, fma(A1, u[1].cm, u[1].y));
-        synth_next_m(u[0], sect_next);
-        synth_next_m(u[1], sect_next);
-        ++m;
-        if (HALVES && NW == 4 && m == mid) {
-          first[0] = u[0].y;
-          first[1] = u[1].y;
-          u[0].y = u[1].y = T(0);
+        for (int k = 0; k < G; ++k) {
+          const T be = T(cur[3 * k]), cc = T(cur[3 * k + 1]), ss = T(cur[3 * k + 2]);
+          const T p = fma(u[0].mu, p1, be * p2);
+          const T r = fma(u[1].mu, r1, be * r2);
+          p2 = p1;
+          p1 = p;
+          r2 = r1;
+          r1 = r;
+          A0 = fma(cc, p, A0);
+          B0 = fma(ss, p, B0);
+          A1 = fma(cc, r, A1);
+          B1 = fma(ss, r, B1);
         }
-        left = (L - m + G) / G;
-        sect_next = sect[min(m + 1, L)];
-        A0 = B0 = A1 = B1 = T(0);
-        p1 = r1 = T(0);
-        p2 = u[0].pmm;
-        r2 = u[1].pmm;
+        if (--left == 0) {
+          u[0].y = fma(B0, u[0].sm, fma(A0, u[0].cm, u[0].y));
+          u[1].y = fma(B1, u[1].sm, fma(A1, u[1].cm, u[1].y));
+          synth_next_m(u[0], sect_next);
+          synth_next_m(u[1], sect_next);
+          ++m;
+          left = (L - m + G) / G;
+          sect_next = sect[min(m + 1, L)];
+          A0 = B0 = A1 = B1 = T(0);
+          p1 = r1 = T(0);
+          p2 = u[0].pmm;
+          r2 = u[1].pmm;
+        }
+      }
+      if constexpr (kHalves == 2) {  // the lane's own entries
+        const double y0 = u[0].y, y1 = u[1].y;
+        u[0].y = half ? part[0][threadIdx.x] + y0 : 0.0;
+        u[1].y = half ? part[1][threadIdx.x] + y1 : 0.0;
+        part[0][threadIdx.x] = y0;
+        part[1][threadIdx.x] = y1;
       }
     }
-  }
-  if (HALVES && NW == 4) {
-    u[0].y = first[0] + u[0].y;
-    u[1].y = first[1] + u[1].y;
   }
   part[0][threadIdx.x] = double(u[0].y);
   part[1][threadIdx.x] = double(u[1].y);
@@ -1828,7 +1830,9 @@ __global__ __launch_bounds__(64 * NW) void k_sh_synth_chain(int L, int N, const 
 // degree 8, 642 4.8 / 4.3 (nine orders do not fill eight waves).  Eight ranges
 // are cut either way and the sums are the same bit for bit: four waves run two
 // ranges each, one sum after the other, and of eight waves the odd ones rotate
-// from the start of the range before theirs, as that wave would.
+// from the start of the range before theirs, as that wave would.  (Two sums
+// instead of one cost four waves 0.5 us at 163842 cells, degrees 16 and 32;
+// starting each range by binary powers cost 2.4.)
 constexpr unsigned int kSynthWideBelow = 768;
 
 // Orders of the NW ranges of the chain synthesis: near-equal costs, order m
@@ -3589,10 +3593,14 @@ static int sh_apply(odis_ctx *ctx, const T *x, long long stride, int nb, const d
     hipEvent_t e4 = ev ? ev[4] : nullptr, e5 = ev ? ev[5] : nullptr;
     if (by_pair) {
       // FP32 contexts keep the order of their sums (see pair_degree)
-      const bool eight = sizeof(T) == 8 && L > 8, wide = eight && gs2.x * nb < kSynthWideBelow;
-      const SynthCuts cut = sizeof(T) == 8 ? chain_split(L, eight ? 8 : 4) : SynthCuts{{0, mr.x, mr.y, mr.z, mr.w}};
-      auto *const kernel = !eight ? &k_sh_synth_chain<T, 4, false>
-                                  : (wide ? &k_sh_synth_chain<T, 8, true> : &k_sh_synth_chain<T, 4, true>);
+      auto *kernel = &k_sh_synth_chain<T, 4, false>;
+      SynthCuts cut{{0, mr.x, mr.y, mr.z, mr.w}};
+      bool wide = false;
+      if constexpr (sizeof(T) == 8) {
+        wide = L > 8 && gs2.x * nb < kSynthWideBelow;
+        if (L > 8) kernel = wide ? &k_sh_synth_chain<T, 8, true> : &k_sh_synth_chain<T, 4, true>;
+        cut = chain_split(L, L > 8 ? 8 : 4);
+      }
       hipExtLaunchKernelGGL(kernel, gs2, dim3(wide ? 512 : 256), 0, ctx->stream, e4, e5, 0, L, N, ctx->sh_tabm,
                             ctx->sh_chain, ctx->sh_trig, ctx->sh_cmaj, base, stride, out, cut);
     }
