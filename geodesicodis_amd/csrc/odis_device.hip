@@ -1745,7 +1745,6 @@ __global__ __launch_bounds__(64 * NW) void k_sh_synth_chain(int L, int N, const 
     u[h].pmm = T(1);
     u[h].y = T(0);
   }
-  T first[2] = {T(0), T(0)};
   if (mlo < mhi) {
     const double *e = cmaj + size_t(b) * 3 * chain_at(L, L + 1) + 3 * chain_at(L, mlo);
     if constexpr (sizeof(T) == 8) {
@@ -4299,7 +4298,7 @@ struct ResOrder {
       v->erase(std::remove_if(v->begin(), v->end(), [ctx](const Member &m) { return m.ctx == ctx; }), v->end());
   }
 };
-static ResOrder g_res_order[16];
+static ResOrder *const g_res_order = new ResOrder[16];  // per device; a context may end after main
 static void res_forget(odis_ctx *ctx) { g_res_order[ctx->res.dev & 15].forget(ctx); }
 
 // Enqueue `count` steps of every instance from ctx->step in one launch.
