@@ -1732,6 +1732,8 @@ __global__ __launch_bounds__(64 * NW) void k_sh_synth_chain(int L, int N, const 
   // orders [mlo, mhi); the rotation starts at mst, the second sum at mid
   const int mlo = cut.m[kHalves * g], mhi = cut.m[kHalves * (g + 1)], mid = cut.m[kHalves * g + 1];
   const int mst = HALVES && NW == 8 ? cut.m[g & ~1] : mlo;
+  double turn = 0.0;
+  if constexpr (HALVES && NW == 8) turn = sect[min(mst + 1 + lane, L)];
   SynthCell<T> u[2];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
@@ -1752,9 +1754,17 @@ __global__ __launch_bounds__(64 * NW) void k_sh_synth_chain(int L, int N, const 
       synth_start(u[0], mst, cmm);
       synth_start(u[1], mst, cmm);
     }
-    for (int q = sizeof(T) == 8 ? mst + 1 : 1; q <= mlo; ++q) {
-      synth_next_m(u[0], sect[q]);
-      synth_next_m(u[1], sect[q]);
+    if constexpr (HALVES && NW == 8) {  // lane k holds the factor of order mst + 1 + k
+      for (int q = 0; q < mlo - mst; ++q) {
+        const double f = lane_value(turn, q);
+        synth_next_m(u[0], f);
+        synth_next_m(u[1], f);
+      }
+    } else if constexpr (sizeof(T) == 4) {
+      for (int q = 1; q <= mlo; ++q) {
+        synth_next_m(u[0], sect[q]);
+        synth_next_m(u[1], sect[q]);
+      }
     }
     T A0 = T(0), B0 = T(0), A1 = T(0), B1 = T(0);
     T p1 = T(0), p2 = u[0].pmm, r1 = T(0), r2 = u[1].pmm;

@@ -1,9 +1,11 @@
 """Resident runs of few steps, as asynchronous calls make them behind a longer
 one: the same state bit for bit as the same steps launched one by one."""
+import threading
+
 import numpy as np
 import pytest
 
-from test_gpu_resident import _ocean, _pair, _same
+from test_gpu_resident import KEYS, _ocean, _pair, _same
 
 pytestmark = pytest.mark.gpu
 
@@ -76,4 +78,44 @@ def test_a_launch_taken_back(product, level, precision, n, miss, stride):
     for i in (0, n - 1):
         assert np.allclose(a.dissipation_series(i, 0, done), b.dissipation_series(i, 0, done), rtol=1e-12, atol=0)
     for c in (a, b):
+        c.close()
+
+
+def test_launches_side_by_side(product):
+    """Contexts of several sizes stepping from threads of their own, their
+    launches beside and behind each other: each ends as it does alone, and none
+    of them is taken back."""
+    G = product
+    runs = []
+    for level, option, steps in [(4, 1, 37), (4, 1, 40), (5, 1, 25), (6, 200, 30), (6, 1, 20), (5, 50, 33), (4, 3, 50),
+                                 (7, 1, 15)]:
+        mesh, ps, start = _ocean(G, level, 1)
+        c = G.Context(mesh, ps)
+        c.set_option(G.OPT_RESIDENT, option)
+        c.set_state(v=start[0][0], eta=start[0][1])
+        runs.append((c, mesh, start[0], steps))
+    want = []
+    for c, mesh, (v, eta), steps in runs:
+        for _ in range(12):
+            c.step(steps)
+        want.append(c.get_state())
+        c.set_state(v=v, eta=eta, dvdt=np.zeros((mesh.E, 3)), detadt=np.zeros((mesh.N, 3)))
+
+    def go(c, steps):
+        for k in range(12):
+            c.step(steps, sync=False)
+            if k % 5 == 4:
+                c.sync()
+        c.sync()
+    th = [threading.Thread(target=go, args=(c, steps)) for c, _, _, steps in runs]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join(60)
+        assert not t.is_alive()
+    for (c, _, _, _), w in zip(runs, want):
+        assert c.option(G.OPT_RESIDENT_ACTIVE) > 0
+        got = c.get_state()
+        for k in KEYS:
+            assert np.array_equal(got[k], w[k]), k
         c.close()
