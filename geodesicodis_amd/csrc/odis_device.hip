@@ -1252,94 +1252,92 @@ __global__ __launch_bounds__(64 * kShWaves) void k_sh_analysis_rec(int L, int N,
   // lane of sum q after reduce_scatter16 is rev4(q); this lane holds q = rev4(lane & 15)
   const int q_lane = ((lane & 1) << 3) | ((lane & 2) << 1) | ((lane & 4) >> 1) | ((lane & 8) >> 3);
   if (chunk < n_chunks) {
-    {
-      double *slot = rw;
-      int oab = 2 * (L + 1);
-      for (int q = 0; q < m; ++q) oab += 2 * max(0, L - q - 1);
-      const double *ab = tabm + oab;  // (a, b) of l = m + 2 + j at 2 j
-      // every cell's operands are under way before the first is used, and a
-      // table entry is loaded once for all of them (one cell after the other,
-      // each waiting for its loads and m table entries: 17.6 us at 10242 cells,
-      // degree 12, instead of 13.9)
-      T mu[CPT], xc[CPT], xs[CPT], p1[CPT], p2[CPT], s[CPT], cl[CPT], sl[CPT];
+    double *slot = rw;
+    int oab = 2 * (L + 1);
+    for (int q = 0; q < m; ++q) oab += 2 * max(0, L - q - 1);
+    const double *ab = tabm + oab;  // (a, b) of l = m + 2 + j at 2 j
+    // every cell's operands are under way before the first is used, and a
+    // table entry is loaded once for all of them (one cell after the other,
+    // each waiting for its loads and m table entries: 17.6 us at 10242 cells,
+    // degree 12, instead of 13.9)
+    T mu[CPT], xc[CPT], xs[CPT], p1[CPT], p2[CPT], s[CPT], cl[CPT], sl[CPT];
+#pragma unroll
+    for (int j = 0; j < CPT; ++j) {
+      const int i = min((chunk * CPT + j) * 64 + lane, N - 1);
+      mu[j] = T(trig[i]);
+      s[j] = T(trig[N + i]);
+      cl[j] = T(trig[2 * N + i]);
+      sl[j] = T(trig[3 * N + i]);
+      p2[j] = xb[i];  // x, until the chain starts
+    }
+#pragma unroll
+    for (int j = 0; j < CPT; ++j) {
+      if ((chunk * CPT + j) * 64 + lane >= N) {
+        mu[j] = s[j] = sl[j] = p2[j] = T(0);
+        cl[j] = T(1);
+      }
+      xc[j] = T(1);   // cos, sin (m lon)
+      xs[j] = T(0);
+      p1[j] = T(1);   // P_mm
+    }
+    for (int q = 1; q <= m; ++q) {
+      const T sect = T(tsect[q]);
 #pragma unroll
       for (int j = 0; j < CPT; ++j) {
-        const int i = min((chunk * CPT + j) * 64 + lane, N - 1);
-        mu[j] = T(trig[i]);
-        s[j] = T(trig[N + i]);
-        cl[j] = T(trig[2 * N + i]);
-        sl[j] = T(trig[3 * N + i]);
-        p2[j] = xb[i];  // x, until the chain starts
+        const T c2 = fma(xc[j], cl[j], -(xs[j] * sl[j]));
+        xs[j] = fma(xs[j], cl[j], xc[j] * sl[j]);
+        xc[j] = c2;
+        p1[j] = p1[j] * (sect * s[j]);
       }
+    }
 #pragma unroll
-      for (int j = 0; j < CPT; ++j) {
-        if ((chunk * CPT + j) * 64 + lane >= N) {
-          mu[j] = s[j] = sl[j] = p2[j] = T(0);
-          cl[j] = T(1);
-        }
-        xc[j] = T(1);   // cos, sin (m lon)
-        xs[j] = T(0);
-        p1[j] = T(1);   // P_mm
-      }
-      for (int q = 1; q <= m; ++q) {
-        const T sect = T(tsect[q]);
+    for (int j = 0; j < CPT; ++j) {
+      xc[j] = p2[j] * xc[j];
+      xs[j] = p2[j] * xs[j];
+      p2[j] = T(0);  // p1: P_{l-1} for l = m + 1 after the first degree
+    }
+    const int nl = L - m + 1;  // degrees m .. L, index t = l - m
+    const T f = T(tf1[m]);
+    for (int t0 = 0; t0 < nl; t0 += 8) {
+      T v[16];
 #pragma unroll
-        for (int j = 0; j < CPT; ++j) {
-          const T c2 = fma(xc[j], cl[j], -(xs[j] * sl[j]));
-          xs[j] = fma(xs[j], cl[j], xc[j] * sl[j]);
-          xc[j] = c2;
-          p1[j] = p1[j] * (sect * s[j]);
-        }
-      }
+      for (int u = 0; u < 8; ++u) {
+        const int t = t0 + u;  // wave-uniform
+        T ac = T(0), as = T(0);
+        if (t < nl) {
+          if (t == 0) {
 #pragma unroll
-      for (int j = 0; j < CPT; ++j) {
-        xc[j] = p2[j] * xc[j];
-        xs[j] = p2[j] * xs[j];
-        p2[j] = T(0);  // p1: P_{l-1} for l = m + 1 after the first degree
-      }
-      const int nl = L - m + 1;  // degrees m .. L, index t = l - m
-      const T f = T(tf1[m]);
-      for (int t0 = 0; t0 < nl; t0 += 8) {
-        T v[16];
+            for (int j = 0; j < CPT; ++j) {
+              ac = fma(p1[j], xc[j], ac);
+              as = fma(p1[j], xs[j], as);
+            }
+          } else if (t == 1) {
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          const int t = t0 + u;  // wave-uniform
-          T ac = T(0), as = T(0);
-          if (t < nl) {
-            if (t == 0) {
+            for (int j = 0; j < CPT; ++j) {
+              const T p = f * mu[j] * p1[j];
+              p2[j] = p1[j];
+              p1[j] = p;
+              ac = fma(p, xc[j], ac);
+              as = fma(p, xs[j], as);
+            }
+          } else {
+            const T a = T(ab[2 * (t - 2)]), bb = T(ab[2 * (t - 2) + 1]);
 #pragma unroll
-              for (int j = 0; j < CPT; ++j) {
-                ac = fma(p1[j], xc[j], ac);
-                as = fma(p1[j], xs[j], as);
-              }
-            } else if (t == 1) {
-#pragma unroll
-              for (int j = 0; j < CPT; ++j) {
-                const T p = f * mu[j] * p1[j];
-                p2[j] = p1[j];
-                p1[j] = p;
-                ac = fma(p, xc[j], ac);
-                as = fma(p, xs[j], as);
-              }
-            } else {
-              const T a = T(ab[2 * (t - 2)]), bb = T(ab[2 * (t - 2) + 1]);
-#pragma unroll
-              for (int j = 0; j < CPT; ++j) {
-                const T p = fma(a * mu[j], p1[j], -(bb * p2[j]));
-                p2[j] = p1[j];
-                p1[j] = p;
-                ac = fma(p, xc[j], ac);
-                as = fma(p, xs[j], as);
-              }
+            for (int j = 0; j < CPT; ++j) {
+              const T p = fma(a * mu[j], p1[j], -(bb * p2[j]));
+              p2[j] = p1[j];
+              p1[j] = p;
+              ac = fma(p, xc[j], ac);
+              as = fma(p, xs[j], as);
             }
           }
-          v[2 * u] = ac;
-          v[2 * u + 1] = as;
         }
-        const T r = reduce_scatter16(v, lane);
-        // lane with (lane & 15) = rev4(q) writes sum q = 2 u + s: degree t0 + u
-        if (lane < 16 && t0 + (q_lane >> 1) < nl) slot[2 * t0 + q_lane] = double(r);
+        v[2 * u] = ac;
+        v[2 * u + 1] = as;
       }
+      const T r = reduce_scatter16(v, lane);
+      // lane with (lane & 15) = rev4(q) writes sum q = 2 u + s: degree t0 + u
+      if (lane < 16 && t0 + (q_lane >> 1) < nl) slot[2 * t0 + q_lane] = double(r);
     }
   }
   __syncthreads();
@@ -1839,9 +1837,9 @@ __global__ __launch_bounds__(64 * NW) void k_sh_synth_chain(int L, int N, const 
 // degree 8, 642 4.8 / 4.3 (nine orders do not fill eight waves).  Eight ranges
 // are cut either way and the sums are the same bit for bit: four waves run two
 // ranges each, one sum after the other, and of eight waves the odd ones rotate
-// from the start of the range before theirs, as that wave would.  (Two sums
-// instead of one cost four waves 0.5 us at 163842 cells, degrees 16 and 32;
-// starting each range by binary powers cost 2.4.)
+// from the start of the range before theirs, as that wave would.  It costs 0.5
+// us: 163842 cells, degrees 16 and 32 (two sums in four waves; with a start of
+// its own for each range 2.4), and 40962 cells, degree 32 (the rotations).
 constexpr unsigned int kSynthWideBelow = 768;
 
 // Orders of the NW ranges of the chain synthesis: near-equal costs, order m
@@ -2477,9 +2475,10 @@ static int upload(odis_ctx *ctx, T **p, const std::vector<T> &h) {
 // contexts: a call takes one and gives it back when it returns (its kernels
 // have finished by then), so there are as many as calls at one time.  At most
 // kStageKeep are kept for later calls, and none once the last context is
-// destroyed.  Small on purpose: the GPU's first accesses to pinned pages after
-// the page tables changed are slow (a 21 MB buffer cost the first call on a
-// new context 10 ms), so a large output goes through the same few pages.
+// destroyed.  Small on purpose: the GPU's first accesses to a new pinned buffer
+// are slow (of 21 MB 10 ms; of this one 1 ms in the first state of 40962 or
+// 163842 cells read after the process had no context), so a large output goes
+// through the same few pages.
 constexpr size_t kStageDoubles = size_t(1) << 18;  // 2 MB
 constexpr size_t kStageKeep = 4;
 struct StagePool {
@@ -5551,10 +5550,10 @@ extern "C" int odis_sh_project(odis_ctx *ctx, const double *field, double *coeff
 }
 
 // ---------------------------------------------------------------------------
-// Projection that allocates nothing.  odis_sh_project allocates the field in
-// device order and the coefficients per call; odis_sh_project_noalloc keeps
-// both in `scratch`, a file-scope device array of kNoAllocScratch doubles
-// (8 MiB per GPU, held until the process ends): [0, N) the field as given,
+// Projection without the basis' scratch and the pinned stage, which
+// odis_sh_project may have to allocate: odis_sh_project_noalloc keeps the field
+// in device order and the coefficients in `scratch`, a file-scope device array
+// of kNoAllocScratch doubles (8 MiB per GPU, held until the process ends): [0, N) the field as given,
 // [N, 2N) the field in device order, [2N, 2N + K) the coefficients.  It
 // rejects 2N + K > kNoAllocScratch.  Host code never uses the array's name
 // as an address: each device's address comes from hipGetSymbolAddress, once

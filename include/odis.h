@@ -128,7 +128,10 @@ int odis_get_state(odis_ctx *ctx, int inst, double *v, double *dvdt, double *eta
 
 /* Advance every instance n_steps iterations of the ab3Explicit loop body
  * (src/timeIntegrator.cpp:207-277).  Stream-ordered; returns after enqueueing
- * unless ODIS_SYNC is set in flags. */
+ * unless ODIS_SYNC is set in flags.  It waits for earlier work where a buffer
+ * of forcing coefficients is still in use (calls more than two ahead), and
+ * where steps launched singly follow a resident run: steps sampled for timing,
+ * and the fourth of several calls of fewer than 4 steps in a row. */
 #define ODIS_SYNC 1
 int odis_step(odis_ctx *ctx, int n_steps, int flags);
 int odis_sync(odis_ctx *ctx);
@@ -359,7 +362,11 @@ int odis_get_option(odis_ctx *ctx, int option, int *value);
  * odis_step call.  T = 0 disables.  odis_enable_timing creates the events a
  * chunk of steps needs; the events are read (waiting for the stream) when
  * odis_get_timing or odis_get_kernel_times asks for them, or when the next
- * odis_step starts, so a timed odis_step adds no host work of its own. */
+ * odis_step starts.  Steps that are not sampled run as without timing where
+ * T leaves room for it: a resident run ends before a sampled step, which then
+ * waits for it (T >= 8; T >= 16 for a batch held interleaved, whose state is
+ * converted around the sampled step; with a smaller T all steps are launched
+ * singly). */
 int odis_enable_timing(odis_ctx *ctx, int stride);
 int odis_get_timing(odis_ctx *ctx, double *face_ms, double *cell_ms, double *step_ms);
 /* The same averages and those of the SH kernels of sampled steps, indexed
