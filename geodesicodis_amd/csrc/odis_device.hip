@@ -4288,14 +4288,16 @@ static int res_setup(odis_ctx *ctx) {
 // workgroups together are no more than the CUs, and a launch that does not fit
 // the newest group begins another, whose launches all start after those of the
 // group before.  (If each workgroup in flight has used up a CU, the CUs left are
-// still as many as the group's workgroups to come.)  A launch begins when the
-// last ones of the group before have ended, and so those of all earlier groups.
+// still as many as the group's workgroups to come.  That has to hold on each
+// XCD: workgroups go round the eight of them, so a launch counts as if it had a
+// multiple of eight.)  A launch begins when the last ones of the group before
+// have ended, and so those of all earlier groups.
 // Eight contexts of 642 cells stepped by eight threads: 21 us per step of all
 // when the launches follow one another, 8.2 so (18.5 launched singly).
 struct ResOrder {
   struct Member {
     const odis_ctx *ctx;
-    unsigned grid;
+    unsigned cus;   // its workgroups, rounded up to the XCDs
     hipEvent_t ev;  // after its last launch in the group
   };
   std::mutex mu;
@@ -4377,8 +4379,9 @@ static int launch_resident(odis_ctx *ctx, Ops<T> &o, const double *table, int co
     std::lock_guard<std::mutex> lock(ord.mu);
     const auto own = [ctx](const ResOrder::Member &m) { return m.ctx == ctx; };
     if (std::none_of(ord.group.begin(), ord.group.end(), own)) {
-      unsigned all = grid;
-      for (const auto &m : ord.group) all += m.grid;
+      const unsigned cus = (grid + 7) / 8 * 8;
+      unsigned all = cus;
+      for (const auto &m : ord.group) all += m.cus;
       if (all > unsigned(r.n_cu) && !ord.group.empty()) {
         ord.before = std::move(ord.group);
         ord.group.clear();
@@ -4386,7 +4389,7 @@ static int launch_resident(odis_ctx *ctx, Ops<T> &o, const double *table, int co
       for (const auto &m : ord.before)  // (its own is before it in its stream)
         if (m.ctx != ctx) CK(hipStreamWaitEvent(ctx->stream, m.ev, 0));
       r.ev_next ^= 1;  // the other event still stands for the group before
-      ord.group.push_back({ctx, grid, r.ev[r.ev_next]});
+      ord.group.push_back({ctx, cus, r.ev[r.ev_next]});
     }
     void *params[] = {&a};
     CK(hipLaunchKernel(res_kernel<T>(ctx, r.variant), dim3(grid), dim3(lanes), params, lds, ctx->stream));

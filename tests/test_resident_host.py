@@ -248,7 +248,7 @@ def test_launches_of_several_contexts_are_ordered_only_where_they_must_be(stub):
     assert [waits(c) for c in small + small] == [0] * 16
     for c in small:
         c.close()
-    a, x, z, v = context(200), context(100), context(150), context(2)
+    a, x, z, v = context(200), context(96), context(144), context(2)
     assert waits(a) == 0
     assert waits(x) == 1                         # after a
     assert waits(z) == 1                         # beside x, after a
@@ -267,6 +267,24 @@ def test_launches_of_several_contexts_are_ordered_only_where_they_must_be(stub):
     y = ocean(40)                                # more workgroups than compute units
     assert waits(y) == 4
     assert waits(x) == 1
+    """)
+
+
+def test_launches_side_by_side_fit_each_part_of_the_chip(stub):
+    """A launch's workgroups go round the chip's eight parts: one of 33 may put
+    five on any of them, so seven such launches do not fit parts of 32 compute
+    units, though their 231 workgroups are fewer than the 256 units."""
+    stub("""
+    g = mesh(6)
+    p = G.make_params(time_step=1.0)[0]
+    cs = [G.Context(g, [p]) for _ in range(7)]
+    waits = []
+    for c in cs:
+        c.set_option(G.OPT_RESIDENT, 33)
+        log()
+        c.step(8, sync=False)
+        waits.append(sum(x == "after another launch" for x in log()))
+    assert waits == [0] * 6 + [6], waits
     """)
 
 
